@@ -408,7 +408,7 @@ def bench_induct(args):
     """The keys-and-locks producer (`_induct_raw`, full2.py:1499-1535; locks = 3, the longest firing lock kept)
     on the token texts of the configuration (config 2: 32 texts x 1024 tokens; --induct-len T: 32 texts of T tokens
     drawn the same way, e.g. the 16384 of pg19_needle.py:177), timed with torch events on the current stream. It is
-    a per-text sort in LDS (above 8192 tokens, over a workspace with LDS chunk rounds): the HBM roofline is reported
+    a per-text hash table and a walk over the text's chunks (above 8192 tokens, tables in a workspace): the HBM roofline is reported
     for its algorithmic bytes (x in, cand / on / bk out: 8 + 24 + 3 + 8 bytes per token), not as its bound."""
     from memarch_amd import _lib, induct
     from memarch_amd.workloads import CONFIGS, scaled, token_stream
@@ -438,12 +438,12 @@ def bench_induct(args):
         "data": f"synthetic (seeded config {cfg.index} token texts)",
         "config": {"workload": f"_induct_raw on config {cfg.index}'s texts", "texts": int(x.shape[0]),
                    "seq": int(x.shape[1]), "locks": 3},
-        "roofline": {"bound": "hbm", "kernel": "k_induct" if x.shape[1] <= 8192 else "k_induct_long",
+        "roofline": {"bound": "hbm", "kernel": "k_induct" if x.shape[1] <= 8192 else "k_ind_link",
                      "achieved": round(nbytes / dt / 1e9, 2),
                      "peak": PEAK_HBM / 1e9, "unit": "GB/s", "frac": round(nbytes / dt / PEAK_HBM, 6),
                      "bytes_per_launch": nbytes, "traffic": None,
-                     "note": "LDS sort bound: one workgroup per text" if x.shape[1] <= 8192 else
-                             "sort bound: one workgroup per text, wide stages over its workspace in L2"},
+                     "note": "latency bound: one workgroup per text" if x.shape[1] <= 8192 else
+                             "latency bound: one wave walks a text per lock"},
     }
     if args.cpu_rows > 0:
         # all texts of the configuration, repeated until about 2 s of CPU work have been timed

@@ -11,7 +11,7 @@
  *   on[b,t,k]   = [last exists], and with `longest` only the longest lock that fires stays on (full2.py:1528-1530)
  *   bk[b,t]     = bucket[min(x[b,t], nbucket-1)] (the rarity bucket of full2.py:1513), 0 without a table
  *   c1[b,t]     = sum_k cand*on, or c1_none when no lock is on (the reference uses 0, full2.py:1563)
- * Conventions: x is int64 [B, T] row-major with token ids in [-2^50, 2^50); outputs are int64 (cand, src [B,T,locks];
+ * Conventions: x is int64 [B, T] row-major, any token ids; outputs are int64 (cand, src [B,T,locks];
  * bk, c1 [B,T]) or uint8 0/1 (on [B,T,locks], the layout of a torch.bool tensor); any output may be NULL to skip it.
  * mce_induct takes T <= mce_induct_max_len() (8192, a text held in LDS); mce_induct_ws takes T up to 2^24 on a
  * caller-sized workspace (mce_induct_ws_bytes). Every call is asynchronous on `stream` and allocates nothing.
@@ -46,8 +46,8 @@ MCE_INDUCT_API int mce_induct(const int64_t* x, int64_t B, int64_t T, int locks,
 MCE_INDUCT_API int mce_induct_max_len(void);
 
 /* Workspace bytes mce_induct_ws needs for B texts of T tokens: 0 when T <= mce_induct_max_len() (no workspace); above
- * it, per text, 12 bytes per position of T rounded up to a power of two (sort keys and positions) plus 4 * locks + 8
- * per position (links and class ids); 0 also for arguments the call rejects (T > 2^24, B <= 0, locks outside 1-3).
+ * it, per text, 12 bytes per position of T rounded up to a power of two plus 4 * locks + 8 per position (hash tables,
+ * then links; slots); 0 also for arguments the call rejects (T > 2^24, B <= 0, locks outside 1-3).
  * No counterpart in the reference. */
 MCE_INDUCT_API size_t mce_induct_ws_bytes(int64_t B, int64_t T, int locks);
 

@@ -4,116 +4,116 @@
 //
 // For every position t of a text and every lock k (0: the token x[t]; 1: the pair (x[t-1], x[t]); 2: the triple
 // (x[t-2], x[t-1], x[t]); missing predecessors are a sentinel that equals no token), last_k[t] is the latest
-// j < t whose key equals t's. The candidate is x[last_k[t] + 1] (causal: last + 1 <= t).
+// j < t whose key equals t's. The candidate is x[last_k[t] + 1] (causal: last + 1 <= t). A position t < k has no
+// complete key: it has no last and is no other position's last, so only positions t >= k are entered below.
 //
-// One workgroup per text, everything in LDS (T <= 8192). Per lock:
-//   1. composite c = key << 13 | t for t < T (padding to a power of two with ~0), so equal keys sort by position;
-//   2. bitonic sort of the composites;
-//   3. last[t] = the position of the previous sorted element when its key is equal, else -1;
-//   4. class id rep[t] = the first position of t's key (pointer jumping along last), which builds the next lock's
-//      key from two class ids: pair(t) = (rep_tok[t-1] or T, rep_tok[t]), triple(t) = (rep_pair[t-1] or T,
-//      rep_tok[t]). Class ids are < T, so every key fits in 51 bits whatever the vocabulary size.
-// The triple decomposition: (x[t-2], x[t-1], x[t]) == (x[j-2], x[j-1], x[j]) iff pair(t-1) == pair(j-1) and
-// x[t] == x[j]; at t = 0 the pair before t is (none, none), which equals no pair(j) (its second part is a token).
-//
-// Longer texts (k_induct_long, T up to 2^24) keep the same steps on a caller-sized workspace in global memory, one
-// workgroup per text: the (key, position) pairs of a lock are sorted by a bitonic network whose wide stages (partner
-// distance >= 4096) run over the text's arrays and whose narrow stages run on 4096-element chunks staged in LDS (the
-// network of every k <= 4096 in one round per chunk, then one round per chunk for each larger k); last[] follows
-// from the sorted order as above, and the class id of a key is the position of the first element of its run in the
-// sorted order (a block-wide scan of run starts instead of pointer jumping). A text's arrays (12 bytes per position
-// of T rounded up to a power of two, plus 4 * locks + 8 per position) stay in L2 for the passes over them.
+// No sort. A hash table gives every key a slot, and "the previous position with the same slot" follows in two steps:
+//   1. insert: each position finds or claims the slot of its key (linear probing; the entry is the claiming position,
+//      whose tokens are compared, so a slot stands for exactly one key whatever the hash does; the table has more
+//      slots than positions, so a probe always ends). One wave takes one chunk of 64 consecutive positions: matching
+//      the slots across its lanes (one ballot per slot bit) gives each lane the previous lane with its key and marks
+//      the first and the last lane of every key in the chunk;
+//   2. link: one wave walks a text's chunks in order over a table of the latest position per slot: a key's first lane
+//      reads it (the previous position, in an earlier chunk), its last lane writes it. A wave's LDS accesses execute
+//      in order, so the walk does not wait for a chunk's reads before the next chunk's: every lane reads and writes,
+//      the ones with nothing to do at a spare entry of their own, since a branch around an access would wait for it.
+// The work is linear in T; the time is the walk (0.06 us per chunk, 0.11 in the long path) and the latencies of the steps around it.
+//   k_induct       T <= 8192: one workgroup per text, tables in LDS (16-bit entries), all locks at once up to 2048
+//                  tokens, one after the other above.
+//   k_ind_*        longer texts, T up to 2^24, on a caller-sized workspace: the insert of all locks and texts over the
+//                  whole GPU on tables in global memory, then the walks (LDS holds the latest positions, 147 KB of
+//                  slots per workgroup; a text with more slots takes several workgroups that each keep to their own
+//                  slots), then the outputs.
+// Measured (3 locks): 32 texts x 1024 tokens 12.3 us, 59.6 with the bitonic sorts this replaced; 4 x 8192 81 us against
+// 440; 4 x 16384 62 us (insert 21, walks 34) against 1082; 1 x 2^20 1.65 ms against 143.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <cstddef>
 
 #include "../../include/mce_induct.h"
 
 namespace {
 
-constexpr int IND_TMAX = 8192;  // positions per text held in LDS
-constexpr int PB = 13;          // position bits of a composite (IND_TMAX = 2^13)
+constexpr int IND_TMAX = 8192;   // positions per text of k_induct
+constexpr int IND_SMALL = 2048;  // up to here all locks' tables fit at once, with the tokens
 constexpr int IND_THREADS_MAX = 1024;
-constexpr int64_t TOK_OFS = int64_t(1) << 50;  // token keys: x + 2^50, in [0, 2^51) for |x| < 2^50
+constexpr int LINK_AHEAD = 8;    // chunks of a walk whose infos and reads are in flight together
+constexpr uint32_t NONE16 = 0xFFFFu;      // empty 16-bit entry / no previous position
+constexpr uint32_t NONE32 = 0xFFFFFFFFu;  // empty 32-bit entry
 
-__device__ __forceinline__ int key_pos(uint64_t c) { return (int)(c & ((1u << PB) - 1)); }
-__device__ __forceinline__ uint64_t key_of(uint64_t c) { return c >> PB; }
-
-// Bitonic sort (ascending) of comp[0, Tp), Tp a power of two; each thread owns elements tid, tid + nt, ...
-__device__ void bitonic_sort(uint64_t* comp, int Tp, int tid, int nt) {
-  for (int k = 2; k <= Tp; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int i = tid; i < Tp; i += nt) {
-        const int p = i ^ j;
-        if (p > i) {
-          const uint64_t a = comp[i], b = comp[p];
-          const bool up = (i & k) == 0;
-          if ((a > b) == up) {
-            comp[i] = b;
-            comp[p] = a;
-          }
-        }
-      }
-      __syncthreads();
-    }
+// Hash of the (k+1)-gram that ends at t (t >= k): multiply-and-fold rounds with odd 64-bit constants (the fractions of
+// the golden ratio, sqrt 2 and sqrt 3).
+__device__ __forceinline__ uint64_t key_hash(const int64_t* __restrict__ x, int t, int k) {
+  uint64_t h = (uint64_t)x[t] * 0x9E3779B97F4A7C15ull;
+  h ^= h >> 32;
+  if (k > 0) {
+    h = (h + (uint64_t)x[t - 1]) * 0x6A09E667F3BCC909ull;
+    h ^= h >> 29;
   }
-}
-
-// After the sort: last[t] for every t < T (the previous position with the same key, or -1).
-__device__ void last_from_sorted(const uint64_t* comp, int T, int16_t* last, int tid, int nt) {
-  for (int i = tid; i < T; i += nt) {
-    const uint64_t c = comp[i];
-    int16_t l = -1;
-    if (i > 0 && key_of(comp[i - 1]) == key_of(c)) l = (int16_t)key_pos(comp[i - 1]);
-    last[key_pos(c)] = l;
+  if (k > 1) {
+    h = (h + (uint64_t)x[t - 2]) * 0xBB67AE8584CAA73Bull;
+    h ^= h >> 32;
   }
-  __syncthreads();
+  h *= 0x9E3779B97F4A7C15ull;
+  return h ^ (h >> 32);
 }
-
-// rep[t] = first position with t's key: follow last[] to its end by pointer jumping (ceil(log2 T) rounds).
-__device__ void class_ids(const int16_t* last, int T, uint16_t* rep, int tid, int nt) {
-  for (int t = tid; t < T; t += nt) rep[t] = (uint16_t)(last[t] >= 0 ? last[t] : t);
-  __syncthreads();
-  for (int span = 1; span < T; span <<= 1) {
-    uint16_t nxt[IND_TMAX / IND_THREADS_MAX];  // elements per thread: T / nt <= 8 (nt = 1024 when T > 1024)
-    int q = 0;
-    for (int t = tid; t < T; t += nt) nxt[q++] = rep[rep[t]];
-    __syncthreads();
-    q = 0;
-    for (int t = tid; t < T; t += nt) rep[t] = nxt[q++];
-    __syncthreads();
+__device__ __forceinline__ bool same_key(const int64_t* __restrict__ x, int a, int b, int k) {
+  // no short circuit: all of a key's loads go out together
+  int64_t d = x[a] ^ x[b];
+  if (k > 0) d |= x[a - 1] ^ x[b - 1];
+  if (k > 1) d |= x[a - 2] ^ x[b - 2];
+  return d == 0;
+}
+// The lanes of `valid` whose v (below 2^bits) equals this lane's.
+__device__ __forceinline__ uint64_t match_lanes(uint32_t v, int bits, uint64_t valid) {
+  uint32_t lo = (uint32_t)valid, hi = (uint32_t)(valid >> 32);
+#pragma unroll 4
+  for (int b = 0; b < bits; ++b) {
+    const uint32_t one = (uint32_t)((int32_t)(v << (31 - b)) >> 31);  // the bit in every position
+    const uint64_t bal = __builtin_amdgcn_ballot_w64(one != 0);
+    lo &= ~((uint32_t)bal ^ one);
+    hi &= ~((uint32_t)(bal >> 32) ^ one);
   }
+  return ((uint64_t)hi << 32) | lo;
 }
+__device__ __forceinline__ int high_bit(uint64_t m) { return 63 - __builtin_clzll(m); }
 
-// The outputs of every position from last_at(k, t) (the previous position with t's k-gram, or -1).
+// Outputs of positions i0, i0 + step, ... of a text (xt: its tokens; row0: its first position's flat index) from
+// last_at(k, t), the previous position with t's k-gram or -1. cand, on and src go out flat over (t, k), so that the
+// lanes of a wave write consecutive elements.
 template <typename LastAt>
-__device__ void emit(const int64_t* __restrict__ xt, int T, int locks, int longest, LastAt last_at,
+__device__ void emit(const int64_t* xt, int64_t row0, int T, int locks, int longest, LastAt last_at,
                      const int64_t* __restrict__ bucket, int64_t nbucket, int64_t c1_none, int64_t* __restrict__ cand,
                      uint8_t* __restrict__ on, int64_t* __restrict__ src, int64_t* __restrict__ bk,
-                     int64_t* __restrict__ c1, int tid, int nt) {
-  const int64_t row0 = (int64_t)blockIdx.x * T;
-  for (int t = tid; t < T; t += nt) {
-    int lst[3] = {-1, -1, -1};
-    for (int k = 0; k < locks; ++k) lst[k] = last_at(k, t);
-    int64_t sum = 0;
-    bool any = false;
-    for (int k = 0; k < locks; ++k) {
-      bool o = lst[k] >= 0;
+                     int64_t* __restrict__ c1, int i0, int step) {
+  if (cand != nullptr || on != nullptr || src != nullptr) {
+    for (int i = i0; i < T * locks; i += step) {
+      const int t = i / locks, k = i - t * locks;
+      const int l = last_at(k, t);
+      bool o = l >= 0;
       if (longest)
-        for (int j = k + 1; j < locks; ++j) o = o && lst[j] < 0;
-      const int64_t s = lst[k] >= 0 ? (int64_t)lst[k] + 1 : 0;
-      const int64_t cv = lst[k] >= 0 ? xt[s] : 0;
-      const int64_t oi = (row0 + t) * locks + k;
-      if (cand != nullptr) cand[oi] = cv;
+        for (int j = k + 1; j < locks; ++j) o = o && last_at(j, t) < 0;
+      const int64_t oi = row0 * locks + i;
+      if (cand != nullptr) cand[oi] = l >= 0 ? xt[l + 1] : 0;
       if (on != nullptr) on[oi] = o ? 1 : 0;
-      if (src != nullptr) src[oi] = s;
-      if (o) {
-        sum += cv;
-        any = true;
-      }
+      if (src != nullptr) src[oi] = l >= 0 ? (int64_t)l + 1 : 0;
     }
-    if (c1 != nullptr) c1[row0 + t] = any ? sum : c1_none;
+  }
+  if (c1 == nullptr && bk == nullptr) return;
+  for (int t = i0; t < T; t += step) {
+    if (c1 != nullptr) {
+      int64_t sum = 0;
+      bool any = false, longer = false;
+      for (int k = locks - 1; k >= 0; --k) {
+        const int l = last_at(k, t);
+        if (l < 0 || (longest && longer)) continue;
+        sum += xt[l + 1];
+        any = longer = true;
+      }
+      c1[row0 + t] = any ? sum : c1_none;
+    }
     if (bk != nullptr) {
       int64_t b = 0;
       if (bucket != nullptr) {
@@ -126,108 +126,103 @@ __device__ void emit(const int64_t* __restrict__ xt, int T, int locks, int longe
   }
 }
 
+// ---------------------------------------------------------------------------------------------------------
+// One workgroup per text. The slot of t's key (hash h) in a table of mask + 1 slots, found or claimed: an entry is the
+// claiming position with 16 bits of its key's hash above, so that nearly every entry of another key is passed without
+// a look at its tokens; an odd step over a power of two of slots visits every one.
+__device__ __forceinline__ uint32_t lds_slot(uint32_t* tab, uint32_t mask, uint64_t h, const int64_t* x, int t, int k) {
+  const uint32_t tag = (uint32_t)(h >> 16) & 0xFFFFu, mine = (tag << 16) | (uint32_t)t;
+  const uint32_t step = (uint32_t)(h >> 40) | 1u;
+  uint32_t s = (uint32_t)(h >> 32) & mask;
+  while (true) {
+    const uint32_t e = atomicCAS(tab + s, NONE32, mine);
+    if (e == NONE32 || (e >> 16 == tag && same_key(x, (int)(e & 0xFFFFu), t, k))) return s;
+    s = (s + step) & mask;
+  }
+}
+
+// TM: the most positions; LP: locks per round; XL: the tokens are kept in LDS too. Info of a position: its slot (below
+// 2 TM <= 2^14), bit 14 set for the first and bit 15 for the last lane of its key in the chunk.
+template <int TM, int LP, bool XL>
 __global__ __launch_bounds__(IND_THREADS_MAX) void k_induct(const int64_t* __restrict__ x, int T, int Tp, int locks,
                                                             int longest, const int64_t* __restrict__ bucket,
                                                             int64_t nbucket, int64_t c1_none,
                                                             int64_t* __restrict__ cand, uint8_t* __restrict__ on,
                                                             int64_t* __restrict__ src, int64_t* __restrict__ bk,
                                                             int64_t* __restrict__ c1) {
-  __shared__ uint64_t comp[IND_TMAX];
-  __shared__ int16_t last[3][IND_TMAX];
-  __shared__ uint16_t rep[2][IND_TMAX];
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int64_t* xt = x + (int64_t)blockIdx.x * T;
+  __shared__ uint32_t tab[LP][2 * TM + 64];  // (and a walk's 64 spare entries)
+  __shared__ uint16_t info[LP][TM];
+  __shared__ uint16_t last[3][TM + 64];
+  __shared__ int64_t xs[XL ? TM : 1];
+  const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, nw = nt >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t* xg = x + (int64_t)blockIdx.x * T;
+  const int64_t* xt = XL ? xs : xg;
+  const int nch = (T + 63) >> 6;
+  const uint32_t mask = 2 * (uint32_t)Tp - 1;
+  const int bits = 32 - __builtin_clz(mask);
+  if constexpr (XL)
+    for (int i = tid; i < T; i += nt) xs[i] = xg[i];
 
-  for (int k = 0; k < locks; ++k) {
-    for (int i = tid; i < Tp; i += nt) {
-      uint64_t c = ~uint64_t(0);
-      if (i < T) {
-        uint64_t key;
-        if (k == 0) {
-          key = (uint64_t)(xt[i] + TOK_OFS);
-        } else {
-          const uint64_t before = i > 0 ? rep[k - 1][i - 1] : (uint64_t)T;  // class of the (k)-gram ending at i-1
-          key = before * (uint64_t)(T + 1) + rep[0][i];
-        }
-        c = (key << PB) | (uint64_t)i;
-      }
-      comp[i] = c;
+  for (int k0 = 0; k0 < locks; k0 += LP) {
+    const int lp = min(LP, locks - k0);
+    for (int q = 0; q < lp; ++q)
+      for (int i = tid; i < 2 * Tp; i += nt) tab[q][i] = NONE32;
+    __syncthreads();
+    for (int it = wave; it < lp * nch; it += nw) {
+      const int q = it / nch, t = (it - q * nch) * 64 + lane, k = k0 + q;
+      const bool ok = t < T && t >= k;
+      uint32_t s = 0;
+      if (ok) s = lds_slot(tab[q], mask, key_hash(xt, t, k), xt, t, k);
+      const uint64_t m = match_lanes(s, bits, __builtin_amdgcn_ballot_w64(ok));
+      const uint64_t below = m & ((uint64_t(1) << lane) - 1);
+      const bool first = ok && below == 0, final = ok && (m >> lane) == 1;
+      info[q][t] = (uint16_t)(s | (first ? 1u << 14 : 0u) | (final ? 1u << 15 : 0u));
+      last[k][t] = (uint16_t)(below != 0 && ok ? (uint32_t)(t - lane + high_bit(below)) : NONE16);
     }
     __syncthreads();
-    bitonic_sort(comp, Tp, tid, nt);
-    last_from_sorted(comp, T, last[k], tid, nt);
-    if (k + 1 < locks && k < 2) class_ids(last[k], T, rep[k], tid, nt);
+    // the tables again, now as the latest position per slot
+    for (int q = 0; q < lp; ++q)
+      for (int i = tid; i < 2 * Tp; i += nt) tab[q][i] = NONE32;
+    __syncthreads();
+    if (wave < lp) {
+      uint32_t* latest = tab[wave];
+      for (int c0 = 0; c0 < nch; c0 += LINK_AHEAD) {
+        uint32_t f[LINK_AHEAD], r[LINK_AHEAD];
+#pragma unroll
+        for (int u = 0; u < LINK_AHEAD; ++u) f[u] = info[wave][min(c0 + u, nch - 1) * 64 + lane];
+#pragma unroll
+        for (int u = 0; u < LINK_AHEAD; ++u) {
+          const uint32_t s = f[u] & 0x3FFFu;
+          r[u] = latest[f[u] & (1u << 14) ? s : 2 * TM + lane];
+          latest[f[u] & (1u << 15) ? s : 2 * TM + lane] = (uint32_t)((c0 + u) * 64 + lane);
+        }
+#pragma unroll
+        for (int u = 0; u < LINK_AHEAD; ++u)
+          last[k0 + wave][c0 + u < nch && (f[u] & (1u << 14)) ? (c0 + u) * 64 + lane : TM + lane] = (uint16_t)r[u];
+      }
+    }
+    __syncthreads();
   }
-
-  emit(xt, T, locks, longest, [&](int k, int t) { return (int)last[k][t]; }, bucket, nbucket, c1_none, cand, on,
+  emit(xt, (int64_t)blockIdx.x * T, T, locks, longest,
+       [&](int k, int t) { return last[k][t] == NONE16 ? -1 : (int)last[k][t]; }, bucket, nbucket, c1_none, cand, on,
        src, bk, c1, tid, nt);
 }
 
 // ---------------------------------------------------------------------------------------------------------
 // Long texts.
 constexpr int64_t IND_LONG_MAX = int64_t(1) << 24;  // positions per text of the long path
-constexpr int LCH = 4096;                           // elements per LDS round of its sort (a power of two)
-constexpr uint32_t PAD_POS = 0xFFFFFFFFu;           // position of the padding elements (key ~0: they sort last)
+constexpr int LINK_BYTES = 144 * 1024;              // LDS of a walk's latest positions
+constexpr int LINK_THREADS = 256, LONG_AHEAD = 32;
+// Info of a position: its slot plus one (at most 2^25 - 1), bit 25 set for the last lane of its key in the chunk, the
+// lane of the previous position with its key in the chunk (its own lane: none) in bits 26-31; 0 for t < k.
+constexpr uint32_t SLOT_MASK = (1u << 25) - 1;
 
-__device__ __forceinline__ bool pair_gt(uint64_t ka, uint32_t pa, uint64_t kb, uint32_t pb) {
-  return ka > kb || (ka == kb && pa > pb);
-}
-// index of the q-th comparator of a stage with partner distance j (a power of two): q with a zero inserted at bit j
-__device__ __forceinline__ int64_t cmp_lo(int64_t q, int64_t j) { return ((q & ~(j - 1)) << 1) | (q & (j - 1)); }
-
-// One compare-exchange stage (k, j) over the whole text in global memory; ascending where bit k of the index is 0.
-__device__ void global_stage(uint64_t* key, uint32_t* pos, int64_t Tp, int64_t k, int64_t j, int tid, int nt) {
-  for (int64_t q = tid; q < Tp / 2; q += nt) {
-    const int64_t i = cmp_lo(q, j), p = i + j;
-    const uint64_t ka = key[i], kb = key[p];
-    const uint32_t pa = pos[i], pb = pos[p];
-    if (pair_gt(ka, pa, kb, pb) == ((i & k) == 0)) {
-      key[i] = kb;
-      key[p] = ka;
-      pos[i] = pb;
-      pos[p] = pa;
-    }
-  }
-  __syncthreads();
-}
-
-// The stages (kk, jj) for kk = k0 .. k1 (powers of two) and every jj < LCH (starting at j0 for kk = k0) on each
-// LCH-element chunk of the text, staged through LDS; the direction of a comparator comes from its global index.
-__device__ void chunk_stages(uint64_t* key, uint32_t* pos, int64_t Tp, int64_t k0, int64_t k1, int64_t j0,
-                             uint64_t* lk, uint32_t* lp, int tid, int nt) {
-  for (int64_t c0 = 0; c0 < Tp; c0 += LCH) {
-    for (int i = tid; i < LCH; i += nt) {
-      lk[i] = key[c0 + i];
-      lp[i] = pos[c0 + i];
-    }
-    __syncthreads();
-    for (int64_t kk = k0; kk <= k1; kk <<= 1) {
-      for (int64_t jj = kk == k0 ? j0 : (kk >> 1 < LCH ? kk >> 1 : LCH >> 1); jj > 0; jj >>= 1) {
-        for (int q = tid; q < LCH / 2; q += nt) {
-          const int i = (int)cmp_lo(q, jj), p = i + (int)jj;
-          const uint64_t ka = lk[i], kb = lk[p];
-          const uint32_t pa = lp[i], pb = lp[p];
-          if (pair_gt(ka, pa, kb, pb) == (((c0 + i) & kk) == 0)) {
-            lk[i] = kb;
-            lk[p] = ka;
-            lp[i] = pb;
-            lp[p] = pa;
-          }
-        }
-        __syncthreads();
-      }
-    }
-    for (int i = tid; i < LCH; i += nt) {
-      key[c0 + i] = lk[i];
-      pos[c0 + i] = lp[i];
-    }
-    __syncthreads();
-  }
-}
-
-// Workspace of one text: key [Tp] u64, pos [Tp] u32, last [locks][T] i32, rep [2][T] i32, each 256-byte aligned.
+// Workspace of one text: the locks' tables, `slots` 32-bit entries each, from the start of the text's part (later
+// the links last[locks][T] i32: the tables are then no longer needed), and the infos [locks][T] u32 at `info`.
 struct LongLayout {
-  size_t pos, last, rep, bytes;
+  size_t info, bytes;
+  uint32_t slots;
 };
 inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 inline int64_t pow2_at_least(int64_t T) {
@@ -235,93 +230,155 @@ inline int64_t pow2_at_least(int64_t T) {
   while (p < T) p <<= 1;
   return p;
 }
+// The size is 12 bytes per position of T rounded up to a power of two, plus 4 * locks + 8 per position; the tables
+// take all of it but the infos, at most 2 slots per padded position: never fewer than 1.66 slots per position.
 LongLayout long_layout(int64_t T, int locks) {
   const size_t tp = (size_t)pow2_at_least(T);
   LongLayout l{};
-  l.pos = align256(8 * tp);
-  l.last = l.pos + align256(4 * tp);
-  l.rep = l.last + align256(4 * (size_t)locks * (size_t)T);
-  l.bytes = l.rep + align256(8 * (size_t)T);
+  const size_t tables = align256(8 * tp) + align256(4 * tp) + align256(8 * (size_t)T);
+  l.info = tables;
+  l.bytes = tables + align256(4 * (size_t)locks * (size_t)T);
+  const size_t slots = std::min(2 * tp, tables / (4 * (size_t)locks));
+  l.slots = (uint32_t)std::min(slots, (size_t)SLOT_MASK - 1);
   return l;
 }
 
-__global__ __launch_bounds__(IND_THREADS_MAX) void k_induct_long(const int64_t* __restrict__ x, int T, int64_t Tp,
-                                                                 int locks, int longest,
-                                                                 const int64_t* __restrict__ bucket, int64_t nbucket,
-                                                                 int64_t c1_none, char* __restrict__ ws,
-                                                                 size_t per_text, size_t off_pos, size_t off_last,
-                                                                 size_t off_rep, int64_t* __restrict__ cand,
-                                                                 uint8_t* __restrict__ on, int64_t* __restrict__ src,
-                                                                 int64_t* __restrict__ bk, int64_t* __restrict__ c1) {
-  __shared__ uint64_t lk[LCH];
-  __shared__ uint32_t lp[LCH];
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int64_t* xt = x + (int64_t)blockIdx.x * T;
-  char* base = ws + (size_t)blockIdx.x * per_text;
-  uint64_t* key = reinterpret_cast<uint64_t*>(base);
-  uint32_t* pos = reinterpret_cast<uint32_t*>(base + off_pos);
-  int32_t* last = reinterpret_cast<int32_t*>(base + off_last);
-  int32_t* rep = reinterpret_cast<int32_t*>(base + off_rep);
-  int* scan = reinterpret_cast<int*>(lk);  // the run-start scan reuses the sort's LDS (IND_THREADS_MAX ints)
+// Empty tables: block (.., text).
+__global__ __launch_bounds__(256) void k_ind_clear(char* __restrict__ ws, size_t per_text, uint32_t entries) {
+  uint32_t* tab = reinterpret_cast<uint32_t*>(ws + (size_t)blockIdx.y * per_text);
+  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < entries; i += gridDim.x * 256) tab[i] = NONE32;
+}
 
-  for (int k = 0; k < locks; ++k) {
-    for (int64_t i = tid; i < Tp; i += nt) {
-      uint64_t kv = ~uint64_t(0);
-      uint32_t pv = PAD_POS;
-      if (i < T) {
-        if (k == 0) {
-          kv = (uint64_t)(xt[i] + TOK_OFS);
-        } else {
-          const uint64_t before = i > 0 ? (uint64_t)rep[(k - 1) * (int64_t)T + i - 1] : (uint64_t)T;
-          kv = before * (uint64_t)(T + 1) + (uint64_t)rep[i];
-        }
-        pv = (uint32_t)i;
-      }
-      key[i] = kv;
-      pos[i] = pv;
+// Slot of t's key (hash h) in a table in global memory, found or claimed. An entry, once set, never changes: the
+// claiming position in bits 0-23 (< 2^24) and 7 bits of its key's hash above, so that nearly every entry of another
+// key is passed without a look at its tokens. The first probes go to independent places (the tables are up to 60%
+// full, where linear probing alone forms long runs, and a wave waits for its slowest lane), the later ones are linear,
+// so that they visit every slot.
+__device__ __forceinline__ uint32_t place(uint32_t h, uint32_t slots) {
+  return (uint32_t)(((uint64_t)h * slots) >> 32);
+}
+__device__ __forceinline__ uint32_t global_slot(uint32_t* tab, uint32_t slots, uint64_t h, const int64_t* __restrict__ x,
+                                                int t, int k) {
+  const uint32_t tag = (uint32_t)(h >> 40) & 0x7Fu, mine = (tag << 24) | (uint32_t)t;
+  uint32_t g = (uint32_t)h, s = place(g, slots);
+  for (int probe = 0;; ++probe) {
+    const uint32_t e = atomicCAS(tab + s, NONE32, mine);
+    if (e == NONE32 || (e >> 24 == tag && same_key(x, (int)(e & 0xFFFFFFu), t, k))) return s;
+    if (probe < 6) {
+      g = g * 0x9E3779B1u + (uint32_t)(h >> 32);
+      s = place(g, slots);
+    } else if (++s == slots) {
+      s = 0;
     }
-    __syncthreads();
-    // every k <= LCH within the chunks, then each larger k: its wide stages over the text, its narrow ones in LDS
-    chunk_stages(key, pos, Tp, 2, LCH, 1, lk, lp, tid, nt);
-    for (int64_t kk = 2 * LCH; kk <= Tp; kk <<= 1) {
-      for (int64_t j = kk >> 1; j >= LCH; j >>= 1) global_stage(key, pos, Tp, kk, j, tid, nt);
-      chunk_stages(key, pos, Tp, kk, kk, LCH >> 1, lk, lp, tid, nt);
-    }
-    // last[k][t]: the previous element of t's run in the sorted order (padding sorts after every real key)
-    int32_t* lastk = last + (int64_t)k * T;
-    for (int64_t i = tid; i < T; i += nt) lastk[pos[i]] = (i > 0 && key[i - 1] == key[i]) ? (int32_t)pos[i - 1] : -1;
-    if (k + 1 < locks && k < 2) {
-      // rep[k][t]: the position of the first element of t's run (the run's smallest position). Each thread takes a
-      // contiguous range of sorted indices; the last run start before a range is the prefix maximum of the run
-      // starts found in the ranges before it.
-      const int64_t per = (T + nt - 1) / nt, s0 = (int64_t)tid * per, s1 = s0 + per < T ? s0 + per : T;
-      int st = -1;
-      for (int64_t i = s0; i < s1; ++i)
-        if (i == 0 || key[i] != key[i - 1]) st = (int)i;
-      scan[tid] = st;
-      __syncthreads();
-      for (int off = 1; off < nt; off <<= 1) {
-        int v = scan[tid];
-        if (tid >= off && scan[tid - off] > v) v = scan[tid - off];
-        __syncthreads();
-        scan[tid] = v;
-        __syncthreads();
-      }
-      int carry = tid > 0 ? scan[tid - 1] : -1;
-      int32_t* repk = rep + (int64_t)k * T;
-      for (int64_t i = s0; i < s1; ++i) {
-        if (i == 0 || key[i] != key[i - 1]) carry = (int)i;
-        repk[pos[i]] = (int32_t)pos[carry];
-      }
-      __syncthreads();
-    }
-    __syncthreads();
   }
-  emit(xt, T, locks, longest, [&](int k, int t) { return (int)last[(int64_t)k * T + t]; }, bucket, nbucket, c1_none,
-       cand, on, src, bk, c1, tid, nt);
+}
+
+// The infos: a wave per (chunk, lock), 4 chunks per block; block (chunk group * locks + lock, text). Lanes that start
+// at the same slot let the lowest of them go first and take its slot where their key is the same, so that a frequent
+// key costs one access of its entry per chunk.
+__global__ __launch_bounds__(256) void k_ind_insert(const int64_t* __restrict__ x, int T, int locks, int bits,
+                                                    char* __restrict__ ws, size_t per_text, size_t off_info,
+                                                    uint32_t slots) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int k = (int)blockIdx.x % locks, t = ((int)blockIdx.x / locks * 4 + wave) * 64 + lane;
+  const int64_t* xt = x + (int64_t)blockIdx.y * T;
+  char* base = ws + (size_t)blockIdx.y * per_text;
+  uint32_t* tab = reinterpret_cast<uint32_t*>(base) + (size_t)k * slots;
+  uint32_t* info = reinterpret_cast<uint32_t*>(base + off_info) + (size_t)k * T;
+  const bool ok = t < T && t >= k;
+  const uint64_t valid = __builtin_amdgcn_ballot_w64(ok);
+  const uint64_t h = ok ? key_hash(xt, t, k) : 0;
+  uint32_t s = place((uint32_t)h, slots);
+  uint64_t m = match_lanes(s, bits, valid);
+  const int lead = ok ? __builtin_ctzll(m) : lane;
+  if (ok && lead == lane) s = global_slot(tab, slots, h, xt, t, k);
+  const uint32_t ls = __shfl(s, lead);
+  // another key that starts at the leader's slot (rare) makes the wave match its lanes again
+  const bool same = lead == lane || (ok && same_key(xt, t - lane + lead, t, k));
+  if (ok && lead != lane) s = same ? ls : global_slot(tab, slots, h, xt, t, k);
+  if (__builtin_amdgcn_ballot_w64(ok && !same) != 0) m = match_lanes(s, bits, valid);
+  const uint64_t below = m & ((uint64_t(1) << lane) - 1);
+  const int prev = below != 0 ? high_bit(below) : lane;
+  if (t < T) info[t] = ok ? (s + 1) | ((m >> lane) == 1 ? 1u << 25 : 0u) | ((uint32_t)prev << 26) : 0u;
+}
+
+// A 32-bit word at byte offset `off` of a buffer of `bytes` bytes: out-of-range offsets load 0 and store nothing, so a
+// walk needs no branch around its accesses.
+typedef __amdgpu_buffer_rsrc_t Rsrc;
+__device__ __forceinline__ Rsrc make_rsrc(void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(p, 0, (int)bytes, 0x00020000);
+}
+
+// The walks: block (part * locks + lock, text) links the positions whose slots are in [part * CAP, (part + 1) * CAP).
+// P: the type of a position (16 bits while every position and the empty mark fit). The first wave walks; the infos of
+// the next LONG_AHEAD chunks are loaded before a batch of chunks is walked, so that the walk (about 0.06 us per chunk)
+// covers their latency.
+template <typename P>
+__global__ __launch_bounds__(LINK_THREADS) void k_ind_link(int T, int locks, char* __restrict__ ws, size_t per_text,
+                                                           size_t off_info) {
+  constexpr uint32_t CAP = LINK_BYTES / sizeof(P);
+  constexpr int LA = LONG_AHEAD;
+  __shared__ __attribute__((aligned(16))) P latest[CAP + 64];  // and the spare entries
+  const int k = (int)blockIdx.x % locks;
+  const uint32_t lo = ((uint32_t)blockIdx.x / (uint32_t)locks) * CAP;
+  char* base = ws + (size_t)blockIdx.y * per_text;
+  const Rsrc info = make_rsrc(base + off_info + 4 * (size_t)k * T, 4 * (uint32_t)T);
+  const Rsrc link = make_rsrc(base + 4 * (size_t)k * T, 4 * (uint32_t)T);
+  for (uint32_t i = threadIdx.x; i < LINK_BYTES / 16; i += LINK_THREADS)
+    reinterpret_cast<uint4*>(latest)[i] = uint4{NONE32, NONE32, NONE32, NONE32};
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  const int lane = threadIdx.x, nch = (T + 63) >> 6;
+  uint32_t nx[LA];
+#pragma unroll
+  for (int u = 0; u < LA; ++u) nx[u] = __builtin_amdgcn_raw_buffer_load_b32(info, (u * 64 + lane) * 4, 0, 0);
+  for (int c0 = 0; c0 < nch; c0 += LA) {
+    uint32_t f[LA], l[LA];
+#pragma unroll
+    for (int u = 0; u < LA; ++u) {
+      f[u] = nx[u];
+      nx[u] = __builtin_amdgcn_raw_buffer_load_b32(info, ((c0 + LA + u) * 64 + lane) * 4, 0, 0);
+    }
+#pragma unroll
+    for (int u = 0; u < LA; ++u) {
+      const uint32_t s = (f[u] & SLOT_MASK) - 1 - lo;
+      const bool mine = f[u] != 0 && s < CAP;
+      l[u] = latest[mine && (int)(f[u] >> 26) == lane ? s : CAP + lane];
+      latest[mine && (f[u] & (1u << 25)) ? s : CAP + lane] = (P)((c0 + u) * 64 + lane);
+    }
+#pragma unroll
+    for (int u = 0; u < LA; ++u) {
+      const int t0 = (c0 + u) * 64, t = t0 + lane, prev = (int)(f[u] >> 26);
+      const bool none = f[u] == 0;
+      const int r = none ? -1 : prev != lane ? t0 + prev : l[u] == (P)NONE32 ? -1 : (int)l[u];
+      // a position without a key (t < k) belongs to the first part
+      const bool mine = none ? lo == 0 : (f[u] & SLOT_MASK) - 1 - lo < CAP;
+      __builtin_amdgcn_raw_buffer_store_b32((uint32_t)r, link, mine ? t * 4 : -4, 0, 0);
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void k_ind_emit(const int64_t* __restrict__ x, int T, int locks, int longest,
+                                                  const int64_t* __restrict__ bucket, int64_t nbucket, int64_t c1_none,
+                                                  const char* __restrict__ ws, size_t per_text,
+                                                  int64_t* __restrict__ cand, uint8_t* __restrict__ on,
+                                                  int64_t* __restrict__ src, int64_t* __restrict__ bk,
+                                                  int64_t* __restrict__ c1, int64_t text0) {
+  const int32_t* last = reinterpret_cast<const int32_t*>(ws + (size_t)blockIdx.y * per_text);
+  const int64_t row0 = (text0 + blockIdx.y) * T;
+  emit(x + (int64_t)blockIdx.y * T, row0, T, locks, longest,
+       [&](int k, int t) { return (int)last[(size_t)k * T + t]; }, bucket, nbucket, c1_none, cand, on, src, bk, c1,
+       (int)blockIdx.x * 256 + (int)threadIdx.x, (int)gridDim.x * 256);
 }
 
 thread_local int g_induct_hip_error = 0;  // the calling thread's last failed launch
+
+int launched() {
+  const hipError_t e = hipGetLastError();
+  if (e == hipSuccess) return MCE_INDUCT_OK;
+  g_induct_hip_error = (int)e;
+  return MCE_INDUCT_ELAUNCH;
+}
 
 }  // namespace
 
@@ -336,16 +393,16 @@ int mce_induct(const int64_t* x, int64_t B, int64_t T, int locks, int longest, c
   if (x == nullptr || B > INT32_MAX) return MCE_INDUCT_EINVAL;
   int Tp = 1;
   while (Tp < T) Tp <<= 1;
-  const int nt = Tp < 64 ? 64 : (Tp > IND_THREADS_MAX ? IND_THREADS_MAX : Tp);
+  // a wave per chunk and lock, as far as a workgroup goes
+  const int nt = (int)std::min<int64_t>(IND_THREADS_MAX, (T + 63) / 64 * 64 * locks);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(k_induct, dim3((unsigned)B), dim3(nt), 0, st, x, (int)T, Tp, locks, longest ? 1 : 0, bucket,
-                     nbucket, c1_none, cand, on, src, bk, c1);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) {
-    g_induct_hip_error = (int)e;
-    return MCE_INDUCT_ELAUNCH;
-  }
-  return MCE_INDUCT_OK;
+  if (T <= IND_SMALL)
+    hipLaunchKernelGGL((k_induct<IND_SMALL, 3, true>), dim3((unsigned)B), dim3(nt), 0, st, x, (int)T, Tp, locks,
+                       longest ? 1 : 0, bucket, nbucket, c1_none, cand, on, src, bk, c1);
+  else
+    hipLaunchKernelGGL((k_induct<IND_TMAX, 1, false>), dim3((unsigned)B), dim3(nt), 0, st, x, (int)T, Tp, locks,
+                       longest ? 1 : 0, bucket, nbucket, c1_none, cand, on, src, bk, c1);
+  return launched();
 }
 
 int mce_induct_max_len(void) { return IND_TMAX; }
@@ -370,15 +427,34 @@ int mce_induct_ws(const int64_t* x, int64_t B, int64_t T, int locks, int longest
   if (need == 0 || ws == nullptr || ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 255))
     return MCE_INDUCT_EINVAL;
   const LongLayout l = long_layout(T, locks);
-  const int64_t Tp = pow2_at_least(T);  // >= 2 * LCH: chunk_stages covers the text in whole chunks
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(k_induct_long, dim3((unsigned)B), dim3(IND_THREADS_MAX), 0, st, x, (int)T, Tp, locks,
-                     longest ? 1 : 0, bucket, nbucket, c1_none, static_cast<char*>(ws), l.bytes, l.pos, l.last, l.rep,
-                     cand, on, src, bk, c1);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) {
-    g_induct_hip_error = (int)e;
-    return MCE_INDUCT_ELAUNCH;
+  int bits = 1;
+  while ((uint32_t(1) << bits) < l.slots) ++bits;
+  const bool small = T < (int64_t)NONE16;  // 16-bit positions
+  const uint32_t cap = LINK_BYTES / (small ? 2 : 4), parts = (l.slots + cap - 1) / cap;
+  const uint32_t entries = l.slots * (uint32_t)locks;
+  const unsigned groups = (unsigned)((T + 255) / 256);
+  const int64_t batch = 32768;  // texts per launch (the grid's second dimension)
+  int rc;
+  for (int64_t b0 = 0; b0 < B; b0 += batch) {
+    const unsigned nb = (unsigned)std::min(batch, B - b0);
+    char* w = static_cast<char*>(ws) + (size_t)b0 * l.bytes;
+    hipLaunchKernelGGL(k_ind_clear, dim3(std::min(1024u, (entries + 1023) / 1024), nb), dim3(256), 0, st, w, l.bytes,
+                       entries);
+    if ((rc = launched())) return rc;
+    hipLaunchKernelGGL(k_ind_insert, dim3(groups * (unsigned)locks, nb), dim3(256), 0, st, x + b0 * T, (int)T, locks,
+                       bits, w, l.bytes, l.info, l.slots);
+    if ((rc = launched())) return rc;
+    if (small)
+      hipLaunchKernelGGL((k_ind_link<uint16_t>), dim3(parts * (unsigned)locks, nb), dim3(LINK_THREADS), 0, st,
+                         (int)T, locks, w, l.bytes, l.info);
+    else
+      hipLaunchKernelGGL((k_ind_link<uint32_t>), dim3(parts * (unsigned)locks, nb), dim3(LINK_THREADS), 0, st,
+                         (int)T, locks, w, l.bytes, l.info);
+    if ((rc = launched())) return rc;
+    hipLaunchKernelGGL(k_ind_emit, dim3(std::min(4096u, groups), nb), dim3(256), 0, st, x + b0 * T, (int)T, locks,
+                       longest ? 1 : 0, bucket, nbucket, c1_none, w, l.bytes, cand, on, src, bk, c1, b0);
+    if ((rc = launched())) return rc;
   }
   return MCE_INDUCT_OK;
 }

@@ -40,7 +40,7 @@ def _launch(x, locks, longest, bucket, c1_none, want):
     if T <= lib.mce_induct_max_len():
         _lib.call("mce_induct", *args, _stream(dev))
     else:
-        # longer texts: the sort runs over a workspace (caching allocator, so 256-byte aligned), freed on return
+        # longer texts: the hash tables lie in a workspace (caching allocator, so 256-byte aligned), freed on return
         # while the kernel may still read it, which the allocator orders by the stream
         nbytes = lib.mce_induct_ws_bytes(B, T, locks)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)

@@ -156,6 +156,42 @@ def test_long_texts_large_token_ids():
     np.testing.assert_array_equal(cand, np.where(si > 0, pool[ci], 0))
 
 
+def _edge_texts(kind, B, T, seed):
+    """one: a single id; two: two ids; distinct: every token once; marked: every other token the same id and the ones
+    between all different (long runs of one token whose pairs and triples never repeat); wide: ids over the whole int64
+    range in repeated blocks."""
+    r = np.random.default_rng(seed)
+    if kind == "one":
+        return np.full((B, T), 5, np.int64)
+    if kind == "two":
+        return r.integers(0, 2, (B, T))
+    if kind == "distinct":
+        return np.stack([r.permutation(T) for _ in range(B)])
+    if kind == "marked":
+        x = np.stack([r.permutation(T) + 1 for _ in range(B)])
+        x[:, ::2] = 0
+        return x
+    pool = r.integers(-(1 << 49), 1 << 49, 64)
+    return pool[np.tile(r.integers(0, 64, (B, 61)), (1, T // 61 + 1))[:, :T]]
+
+
+@pytest.mark.parametrize("T", [3, 63, 65, 129, 2047, 2048, 2049, 4097, 8191, 8193, 16640, 65534, 65535, 73800])
+@pytest.mark.parametrize("kind", ["one", "two", "distinct", "marked", "wide"])
+def test_table_edges_exact(kind, T):
+    """Chunk remainders (64 positions), the lengths where the kernel, the table or the position type changes (2048,
+    8192, 65535), walks over one and several slot ranges, and texts that fill the hash table least and most."""
+    print(f"induct edges {kind} T={T}", flush=True)
+    x = _edge_texts(kind, 2, T, T)
+    ids, rank = np.unique(x, return_inverse=True)     # the oracle runs on ranks: a relabelling keeps every equality
+    rank = rank.reshape(x.shape)
+    cand, on, _, src, c1 = _gpu(x, 3, True)
+    ci, oi, si = io.sorted_scan(rank, len(ids), 3, want_src=True)
+    np.testing.assert_array_equal(on, oi)
+    np.testing.assert_array_equal(src, si)
+    np.testing.assert_array_equal(cand, np.where(si > 0, ids[ci], 0))
+    np.testing.assert_array_equal(c1, io.c1_of(cand, oi, none=-1))
+
+
 @pytest.mark.parametrize("T", [1024, 16384], ids=["lds", "long"])
 def test_no_host_sync_and_graph_capture(T):
     """Both paths issue no host synchronisation (torch.cuda.set_sync_debug_mode("error"), as the loss head is
