@@ -1163,7 +1163,44 @@ __global__ __launch_bounds__(256) void k_row_logits(const uint16_t* __restrict__
   }
 }
 
-// Merge of the T per-half-tile partials: lse, loss, wgt, dgr per row; one loss partial sum per block.
+// Element (m, k) of a tile-blocked [Mp][.] operand (Operand::cm) with Mp rows: the index formula of the layout,
+// with the reduction index k in kperm order.
+__device__ __forceinline__ int64_t cm_index(int64_t m, int64_t k, int64_t Mp) {
+  const int kp = kperm((int)(k & 255));
+  return (k >> 8) * 256 * Mp + (m >> 8) * CM_TILE + ((((m & 255) >> 3) * 32 + (kp >> 3)) * 64) + (m & 7) * 8 +
+         (kp & 7);
+}
+__device__ __forceinline__ uint16_t to_bf16(float x) { return (uint16_t)(pack_bf16x2(x, 0.f) & 0xFFFFu); }
+
+// A training forward's per-row state after the merge (see k_train_rows): G == null: none.
+struct TrainRows {
+  const int64_t* y;
+  const float* lse_est;
+  const int* flag;
+  int64_t Np, Vreal;
+  float* arow;
+  int *flag_count, *flag_list;
+  uint16_t* G;
+};
+// Row n with weight w, lse l and target logit x: a_n and the target's entry; false for a row of the exact pass.
+__device__ __forceinline__ bool train_row(const TrainRows& tr, int64_t n, float w, float l, float x) {
+  const float e = tr.lse_est[n];
+  // every E' value of the row is at most exp(lse - e_n): a row whose lse exceeds e_n by more than 60 also takes
+  // the exact pass (the half-tile bound flags such rows for the logits the tiles see; this catches what they do
+  // not see, the sparse bias)
+  if (tr.flag[n] || !(l - e <= 60.f)) {
+    tr.arow[n] = w;
+    tr.flag_list[atomicAdd(tr.flag_count, 1)] = (int)n;
+    return false;
+  }
+  tr.arow[n] = w * expf(e - l);
+  const int64_t yn = tr.y[n];
+  if (yn >= 0 && yn < tr.Vreal) tr.G[cm_index(n, yn, tr.Np)] = to_bf16(expm1f(x - l) * expf(l - e));
+  return true;
+}
+
+// Merge of the T per-half-tile partials: lse, loss, wgt, dgr per row (and, with tr, train_row: one launch less than a
+// pass of its own, and the row's values are at hand; the grid then covers tr.Np rows).
 // 32 rows per block, 8 threads per row (an online max / rescaled sum over every 8th partial), combined in LDS.
 // With a sparse bias (kc > 0) the tiles saw the logits without it: each distinct valid candidate c then moves
 // its term of the sum from exp(x_c) to exp(x_c + B_c), with the maximum raised first so no term overflows. The
@@ -1177,9 +1214,9 @@ __global__ __launch_bounds__(256) void k_fwd_merge(const float* __restrict__ par
                                                    const float* __restrict__ hit, int64_t N, int T,
                                                    float* __restrict__ loss_rows, float* __restrict__ lse_rows,
                                                    float* __restrict__ wgt_rows, float* __restrict__ dgr_rows,
-                                                   float* __restrict__ loss_part, int* __restrict__ exact_count,
-                                                   int* __restrict__ exact_list) {
-  __shared__ float rm[8][32], rs[8][32], rl[32];
+                                                   int* __restrict__ exact_count, int* __restrict__ exact_list,
+                                                   TrainRows tr) {
+  __shared__ float rm[8][32], rs[8][32];
   const int t = threadIdx.x, r = t & 31, sl = t >> 5;
   const int64_t n = (int64_t)blockIdx.x * 32 + r;
   float m = -INFINITY, s = 0.f;
@@ -1234,8 +1271,10 @@ __global__ __launch_bounds__(256) void k_fwd_merge(const float* __restrict__ par
   rs[sl][r] = s;
   __syncthreads();
   if (sl == 0) {
-    float loss = 0.f;
-    if (n < N) {
+    if (n >= N) {
+      if (tr.G != nullptr && n < tr.Np) tr.arow[n] = 0.f;
+    } else {
+      float loss = 0.f, wgt = 0.f;
       float M = -INFINITY;
 #pragma unroll
       for (int i = 0; i < 8; ++i) M = fmaxf(M, rm[i][r]);
@@ -1269,9 +1308,10 @@ __global__ __launch_bounds__(256) void k_fwd_merge(const float* __restrict__ par
         // (loss_rows == nullptr: only lse is wanted.)
         const bool ok = xy[n] != -INFINITY;
         loss = ok ? d : 0.f;
+        wgt = ok ? 1.f : 0.f;
         if (loss_rows != nullptr) {
           loss_rows[n] = loss;
-          wgt_rows[n] = ok ? 1.f : 0.f;
+          wgt_rows[n] = wgt;
         }
         if (dgr_rows != nullptr) dgr_rows[n] = 0.f;
       } else {
@@ -1284,17 +1324,12 @@ __global__ __launch_bounds__(256) void k_fwd_merge(const float* __restrict__ par
         const float Pc = clamped ? CLAMP_P : P;
         loss = clamped ? -logf(CLAMP_P) : (fabsf(q) < 0.5f ? -log1pf(q) : -logf(P));
         loss_rows[n] = loss;
-        wgt_rows[n] = clamped ? 0.f : (1.f - g) * py / Pc;
+        wgt = clamped ? 0.f : (1.f - g) * py / Pc;
+        wgt_rows[n] = wgt;
         dgr_rows[n] = clamped ? 0.f : (py - h) / Pc;
       }
+      if (tr.G != nullptr) train_row(tr, n, wgt, M + ls, xy[n]);
     }
-    rl[r] = loss;
-  }
-  __syncthreads();
-  if (t == 0 && loss_part != nullptr) {
-    float tot = 0.f;
-    for (int i = 0; i < 32; ++i) tot += rl[i];
-    loss_part[blockIdx.x] = tot;
   }
 }
 
@@ -1385,7 +1420,7 @@ __global__ __launch_bounds__(256) void k_sum_chunks(const float* __restrict__ x,
 // The same sum in one block when count <= SUM_ONE_BLOCK (one launch instead of two): thread t adds values t, t+1024,
 // ... (loads unrolled so that several are in flight), then a fixed-order tree over the 1024 threads.
 constexpr int64_t SUM_ONE_BLOCK = 65536;
-__global__ __launch_bounds__(1024) void k_sum_one(const float* __restrict__ x, int64_t count, float* __restrict__ out) {
+__device__ __forceinline__ void sum_block(const float* __restrict__ x, int64_t count, float* __restrict__ out) {
   __shared__ float red[1024];
   const int t = threadIdx.x;
   float s = 0.f;
@@ -1398,6 +1433,9 @@ __global__ __launch_bounds__(1024) void k_sum_one(const float* __restrict__ x, i
     __syncthreads();
   }
   if (t == 0) out[0] = red[0];
+}
+__global__ __launch_bounds__(1024) void k_sum_one(const float* __restrict__ x, int64_t count, float* __restrict__ out) {
+  sum_block(x, count, out);
 }
 
 __global__ __launch_bounds__(256) void k_sum(const float* __restrict__ part, int64_t count, float* __restrict__ out) {
@@ -1816,15 +1854,6 @@ __global__ __launch_bounds__(256) void k_dgate(const float* __restrict__ dgr, co
 // sum over V of E' W stays far inside the fp32 / bf16 range. A test hook may lower it (mce_train_set_threshold).
 constexpr float TRAIN_S_MAX = 18446744073709551616.f;
 
-// Element (m, k) of a tile-blocked [Mp][.] operand (Operand::cm) with Mp rows: the index formula of the layout,
-// with the reduction index k in kperm order.
-__device__ __forceinline__ int64_t cm_index(int64_t m, int64_t k, int64_t Mp) {
-  const int kp = kperm((int)(k & 255));
-  return (k >> 8) * 256 * Mp + (m >> 8) * CM_TILE + ((((m & 255) >> 3) * 32 + (kp >> 3)) * 64) + (m & 7) * 8 +
-         (kp & 7);
-}
-__device__ __forceinline__ uint16_t to_bf16(float x) { return (uint16_t)(pack_bf16x2(x, 0.f) & 0xFFFFu); }
-
 // chunk_ce on the one-pass path (memarch full2.py:806-830: G = g_lse softmax(x) + g_ly onehot(y), the upstream
 // gradients arriving in the backward). The plain cross-entropy forward left E'[n, v] = exp(x_v - s_n) in G for
 // every v but the target, with s_n = e_n, or s_n = lse_n for a row of the exact pass. Per row this kernel forms
@@ -1991,74 +2020,70 @@ void k_fwd_train(Operand Wop, Operand Hop, const float* __restrict__ bias, const
 
 // After the merge: a_n = wgt_n exp(e_n - lse_n), and the target element of E' in G for unflagged rows,
 // with a sparse bias also the entries of the row's candidates; flagged rows get a_n = wgt_n and are appended to
-// flag_list for the exact pass (k_gather_rows, k_exact_train, k_exact_fix). Rows N .. Np-1 get a_n = 0.
-__global__ __launch_bounds__(256) void k_train_rows(const int64_t* __restrict__ y, const float* __restrict__ xy,
-                                                    const int64_t* __restrict__ cand, const float* __restrict__ cb,
-                                                    const float* __restrict__ xc, int kc,
-                                                    const float* __restrict__ lse_est,
-                                                    const float* __restrict__ lse_rows,
-                                                    const float* __restrict__ wgt_rows, const int* __restrict__ flag,
-                                                    int64_t N, int64_t Np, int64_t Vreal,
-                                                    float* __restrict__ arow, int* __restrict__ flag_count,
-                                                    int* __restrict__ flag_list, uint16_t* __restrict__ G) {
+// flag_list for the exact pass (k_gather_rows, k_exact_train). Rows N .. Np-1 get a_n = 0. Without a sparse bias
+// k_fwd_merge does it itself (with one, the exact lse pass comes in between).
+__global__ __launch_bounds__(256) void k_train_rows(TrainRows tr, const int64_t* __restrict__ cand,
+                                                    const float* __restrict__ cb, const float* __restrict__ xc, int kc,
+                                                    const float* __restrict__ xy, const float* __restrict__ lse_rows,
+                                                    const float* __restrict__ wgt_rows, int64_t N) {
   const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (n >= Np) return;
+  if (n >= tr.Np) return;
   if (n >= N) {
-    arow[n] = 0.f;
+    tr.arow[n] = 0.f;
     return;
   }
-  const float w = wgt_rows[n];
-  const float e = lse_est[n], l = lse_rows[n];
-  // every E' value of the row is at most exp(lse - e_n): a row whose lse exceeds e_n by more than 60 also takes
-  // the exact pass (the half-tile bound flags such rows for the logits the tiles see; this catches what they do
-  // not see, the sparse bias)
-  if (flag[n] || !(l - e <= 60.f)) {
-    arow[n] = w;
-    flag_list[atomicAdd(flag_count, 1)] = (int)n;
-    return;
-  }
-  arow[n] = w * expf(e - l);
-  const int64_t yn = y[n];
-  if (yn >= 0 && yn < Vreal) {
-    G[cm_index(n, yn, Np)] = to_bf16(expm1f(xy[n] - l) * expf(l - e));
-  }
+  const float e = tr.lse_est[n];
+  if (!train_row(tr, n, wgt_rows[n], lse_rows[n], xy[n])) return;
   // sparse bias: each distinct valid candidate other than the target gets its true logit x_c + B_c (the target's
   // x_y already includes its bias)
+  const int64_t yn = tr.y[n];
   for (int k = 0; k < kc; ++k) {
     const int64_t c = cand[n * kc + k];
     const float B = cb[n * kc + k];
     if (c == yn || cb_skip(B)) continue;
-    G[cm_index(n, c, Np)] = to_bf16(expf(xc[n * kc + k] + B - e));
+    tr.G[cm_index(n, c, tr.Np)] = to_bf16(expf(xc[n * kc + k] + B - e));
   }
 }
 
 // The exact E' rows of the flagged rows (rows whose logits exceed e_n by about 44 or more, which a shift by the
-// row's largest known true logit makes rare, or whose lse exceeds e_n by more than 60). Three kernels:
+// row's largest known true logit makes rare, or whose lse exceeds e_n by more than 60). Two kernels:
 // k_gather_rows copies the flagged rows of H into a dense operand Hf [F][K] (F = the flagged-row count); k_exact_train
 // runs the logits tile mainloop over (vocabulary tile, 256 gathered rows) items with each row shifted by its exact
 // lse, so E'[n, v] = exp(x_v - lse_n) (<= 1; a_n = wgt_n for these rows), and stores it in place in G, 16 bytes per
-// lane (the lane's own row); k_exact_fix then writes the target's exp(x_y - lse) - 1 and, with a sparse bias, the
+// lane (the lane's own row), then writes the target's exp(x_y - lse) - 1 and, with a sparse bias, the
 // candidates' exp(x_c + B_c - lse) over those entries. The work is that of F rows of the forward tile pass, so the
 // fallback costs in proportion to the flagged rows. k_exact_train's grid covers every row tile the block could flag
 // (vocabulary tile fastest); a workgroup past the count, read on the device, ends at once, so the pass costs one
 // near-empty launch when nothing is flagged.
 
-// Hf[i, :] = H[list[i], :] for i < *count (K % 8 == 0), 16 bytes per thread, grid-stride.
-__global__ __launch_bounds__(256) void k_gather_rows(const uint16_t* __restrict__ H, int64_t ldh,
-                                                     const int* __restrict__ list, const int* __restrict__ count,
-                                                     int64_t K, uint16_t* __restrict__ Hf) {
-  const int64_t per = K / 8, items = (int64_t)(*count) * per;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < items; i += (int64_t)gridDim.x * 256) {
+// Hf[i, :] = H[list[i], :] for i < *count (K % 8 == 0), 16 bytes per thread, grid-stride. The last block adds up the
+// losses instead (loss_sum not null: the call's last row block, at most SUM_ONE_BLOCK rows), as k_sum_one.
+__global__ __launch_bounds__(1024) void k_gather_rows(const uint16_t* __restrict__ H, int64_t ldh,
+                                                      const int* __restrict__ list, const int* __restrict__ count,
+                                                      int64_t K, uint16_t* __restrict__ Hf,
+                                                      const float* __restrict__ loss_rows, int64_t N,
+                                                      float* __restrict__ loss_sum) {
+  if (blockIdx.x == gridDim.x - 1) {
+    if (loss_sum != nullptr) sum_block(loss_rows, N, loss_sum);
+    return;
+  }
+  const int64_t per = K / 8, items = (int64_t)(*count) * per, step = (int64_t)(gridDim.x - 1) * 1024;
+  for (int64_t i = (int64_t)blockIdx.x * 1024 + threadIdx.x; i < items; i += step) {
     const int64_t r = i / per, c = (i % per) * 8;
     *reinterpret_cast<u16x8*>(Hf + r * K + c) = *reinterpret_cast<const u16x8*>(H + (int64_t)list[r] * ldh + c);
   }
 }
 
+struct ExactFix {   // the rows' known logits (k_row_logits), kc sparse candidates per row
+  const int64_t *y, *cand;
+  const float *xy, *cb, *xc;
+  int kc;
+};
 template <bool KF, bool T16 = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(NTHREADS, NTHREADS), amdgpu_waves_per_eu(1, 1)))
 void k_exact_train(Operand Wop, const uint16_t* __restrict__ Hf, int64_t K, const float* __restrict__ bias,
                    const int* __restrict__ count, const int* __restrict__ list, const float* __restrict__ lse_rows,
-                   int64_t Np, int64_t V, int64_t Vreal, int tiles_v, uint16_t* __restrict__ G) {
+                   int64_t Np, int64_t V, int64_t Vreal, int tiles_v, uint16_t* __restrict__ G, ExactFix fx) {
   __shared__ __attribute__((aligned(1024))) char lds[T16 ? TAIL_OFF + TAIL_BYTES : GRAD_LDS_BYTES];
   const int cnt = *count;
   const int it = (int)blockIdx.x;
@@ -2113,28 +2138,21 @@ void k_exact_train(Operand Wop, const uint16_t* __restrict__ Hf, int64_t K, cons
         }
       }
     }
-  }
-}
-
-// The target and candidate entries of the rows k_exact_train rewrote (list[i], i < *count): E'[n, y_n] =
-// exp(x_y - lse_n) - 1 and, for each distinct valid candidate c != y_n, E'[n, c] = exp(x_c + B_c - lse_n), from the
-// row logits of k_row_logits (x_y with its sparse bias, x_c without), into G. One thread per entry.
-__global__ __launch_bounds__(256) void k_exact_fix(const int* __restrict__ count, const int* __restrict__ list,
-                                                   const int64_t* __restrict__ y, const float* __restrict__ xy,
-                                                   const int64_t* __restrict__ cand, const float* __restrict__ cb,
-                                                   const float* __restrict__ xc, int kc,
-                                                   const float* __restrict__ lse_rows, int64_t Np,
-                                                   int64_t Vreal, uint16_t* __restrict__ G) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= *count) return;
-  const int64_t n = list[i], yn = y[n];
-  const float l = lse_rows[n];
-  if (yn >= 0 && yn < Vreal) G[cm_index(n, yn, Np)] = to_bf16(expm1f(xy[n] - l));
-  for (int k = 0; k < kc; ++k) {
-    const int64_t c = cand[n * kc + k];
-    const float B = cb[n * kc + k];
-    if (c == yn || cb_skip(B)) continue;
-    G[cm_index(n, c, Np)] = to_bf16(expf(xc[n * kc + k] + B - l));
+    // the target and candidate entries of the tile's rows over the stored ones, one thread per row: E'[n, y_n] =
+    // exp(x_y - lse_n) - 1 and, for each distinct valid candidate c != y_n, E'[n, c] = exp(x_c + B_c - lse_n), from
+    // the row logits of k_row_logits (x_y with its sparse bias, x_c without)
+    __threadfence();
+    __syncthreads();
+    if (n0 + t >= cnt) return;
+    const int64_t n = list[n0 + t], yn = fx.y[n];
+    const float l = lse_rows[n];
+    if (yn >= v0 && yn < v0 + BM && yn < Vreal) G[cm_index(n, yn, Np)] = to_bf16(expm1f(fx.xy[n] - l));
+    for (int k = 0; k < fx.kc; ++k) {
+      const int64_t c = fx.cand[n * fx.kc + k];
+      const float B = fx.cb[n * fx.kc + k];
+      if (c == yn || cb_skip(B) || c < v0 || c >= v0 + BM) continue;
+      G[cm_index(n, c, Np)] = to_bf16(expf(fx.xc[n * fx.kc + k] + B - l));
+    }
   }
 }
 
@@ -2183,15 +2201,14 @@ __global__ __launch_bounds__(256) void k_dbias_gemv(const uint16_t* __restrict__
 // reduction index r is stored in the permuted order kperm that G uses for its vocabulary positions (its 16-byte
 // stores), so the products of the dH contraction (W^T) pair up; natural != 0 stores r (and uperm) in natural order
 // instead, the order of G's rows that the dW contraction reduces over (H^T).
-__global__ __launch_bounds__(256) void k_transpose_blocked(const uint16_t* __restrict__ src, int64_t ld, int64_t R,
-                                                           int64_t C, uint16_t* __restrict__ dst,
-                                                           const float* __restrict__ rscale = nullptr,
-                                                           const float* __restrict__ go = nullptr,
-                                                           uint16_t* __restrict__ uperm = nullptr, int natural = 0) {
-  __shared__ __attribute__((aligned(16))) uint16_t tile[64][66];
+typedef uint16_t TransposeTile[64][66];
+__device__ __forceinline__ void transpose_tile(const uint16_t* __restrict__ src, int64_t ld, int64_t R, int64_t C,
+                                               uint16_t* __restrict__ dst, const float* __restrict__ rscale,
+                                               const float* __restrict__ go, uint16_t* __restrict__ uperm, int natural,
+                                               TransposeTile& tile, int bx, int by) {
   const int t = threadIdx.x;
-  const int64_t r0 = (int64_t)blockIdx.x * 64, c0 = (int64_t)blockIdx.y * 64;
-  if (uperm != nullptr && blockIdx.y == 0 && t < 64) {
+  const int64_t r0 = (int64_t)bx * 64, c0 = (int64_t)by * 64;
+  if (uperm != nullptr && by == 0 && t < 64) {
     // the row scales themselves, bf16, in the same order: uperm[r0 + p] = go * rscale[r0 + kperm_inv(p)]
     const int64_t r = r0 + (natural ? t : kperm_inv(t));
     uperm[r0 + t] = r < R ? to_bf16((go != nullptr ? go[0] : 1.f) * rscale[r]) : (uint16_t)0;
@@ -2231,6 +2248,15 @@ __global__ __launch_bounds__(256) void k_transpose_blocked(const uint16_t* __res
       *reinterpret_cast<u16x8*>(dst + (r >> 8) * C * BLK + c * BLK + (r & (BLK - 1))) = v;
     }
   }
+}
+
+__global__ __launch_bounds__(256) void k_transpose_blocked(const uint16_t* __restrict__ src, int64_t ld, int64_t R,
+                                                           int64_t C, uint16_t* __restrict__ dst,
+                                                           const float* __restrict__ rscale = nullptr,
+                                                           const float* __restrict__ go = nullptr,
+                                                           uint16_t* __restrict__ uperm = nullptr, int natural = 0) {
+  __shared__ __attribute__((aligned(16))) TransposeTile tile;
+  transpose_tile(src, ld, R, C, dst, rscale, go, uperm, natural, tile, (int)blockIdx.x, (int)blockIdx.y);
 }
 
 // The bf16 cast of an fp32 weight and its K-blocked transpose in one pass: w16[r, c] = bf16(src[r, c]) (round to
@@ -2287,7 +2313,7 @@ __global__ __launch_bounds__(256) void k_cast_transpose(const float* __restrict_
 // nk_total K stages: s_i = go[0] * rscale[i] (1 for a null go or rscale), Cin an fp32 matrix with C's row stride
 // (null: none; fp32 output only, and it may be C itself, an accumulation). DB > 0 (= fold_nr(tiles_n)):
 // block of tile (tm, tn < 8) also forms sum_k A(m, k) u(k) (u bf16 over the K positions) for the rows m of its
-// 32-row groups tn, tn + tiles_n, .. (DB of them), over its K range: DB 32-value partials per block (k_dbias_tiles
+// 32-row groups tn, tn + tiles_n, .. (DB of them), over its K range: DB 32-value partials per block (dbias_tiles
 // adds them up). The first `full` blocks each compute one whole tile (tiles 0 .. full-1 in the XCD-grouped
 // order). When the tile count leaves a partial last wave on the GPU, the remaining tiles are split along K:
 // block full + r*P + p computes K slice p of P of tile full + r and writes its fp32 partial tile (row-major
@@ -2296,7 +2322,7 @@ __global__ __launch_bounds__(256) void k_cast_transpose(const float* __restrict_
 // most 32), the product of A with the rows of X (the B operand's rows past the tile grid), formed inside the tiles:
 // tile (tm, tn < 8) forms them for its row groups as the dot products above are formed, by one MFMA per group and
 // stage, and writes them with the epilogue below; a K-split tail tile writes its slice's values to
-// xpart[((slot * DB + j) * 32 + i) * 32 + n] (row i of group j, extra column n), which k_xtail_reduce adds up.
+// xpart[((slot * DB + j) * 32 + i) * 32 + n] (row i of group j, extra column n), which xtail_reduce adds up.
 template <bool OUT_BF16, bool KF, int AM, int DB, bool XM = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(NTHREADS, NTHREADS), amdgpu_waves_per_eu(1, 1)))
 void k_gemm(Operand A, Operand B, int nk_total, int64_t M, int64_t Nc, int tiles_m, int tiles_n, int group,
@@ -2456,82 +2482,101 @@ void k_gemm(Operand A, Operand B, int nk_total, int64_t M, int64_t Nc, int tiles
   }
 }
 
+// The K-split tail tiles of one k_gemm launch (full < tiles_m * tiles_n) and what its epilogue needs; xcols > 0: with the
+// extra columns of its XM mode.
+struct TailJob {
+  const float *part, *xpart;
+  int P, full, tails, nr, tiles_m, tiles_n, group, am2, xcols;
+  int64_t M, Nx;
+  void* C;
+  int64_t ldc;
+  const float *rscale, *go, *cin;
+  // blocks: 64 per tail tile (4 rows each), then one per tail tile and row group for the extra columns
+  __host__ __device__ int blocks() const { return tails * (BM / 4 + (xcols > 0 ? nr : 0)); }
+};
+
 // Sum of the P K-slices of each split tail tile into C with k_gemm's epilogue (row scale, Cin) (fixed order
-// p = 0..P-1). Block (group of 4 rows, tile r);
-// thread t sums columns 4*(t%64) .. +3 of row 4*blockIdx.x + t/64 with 16-byte loads.
+// p = 0..P-1). Block (group of 4 rows bx, tail tile r);
+// thread t sums columns 4*(t%64) .. +3 of row 4*bx + t/64 with 16-byte loads, several slices' in flight at a time.
 template <bool OUT_BF16>
-__global__ __launch_bounds__(256) void k_tail_reduce(const float* __restrict__ part, int P, int full, int tiles_m,
-                                                     int tiles_n, int group, int64_t M, int64_t Nc,
-                                                     void* C, int64_t ldc, const float* __restrict__ rscale,
-                                                     const float* __restrict__ go, const float* cin) {
-  const int r = (int)blockIdx.y;
+__device__ __forceinline__ void tail_reduce(const TailJob& j, int bx, int r) {
   int tm, tn;
-  tile_of(full + r, tiles_m, tiles_n, group, tm, tn);
-  const int il = (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6), jl = ((int)threadIdx.x & 63) * 4;
+  tile_of(j.full + r, j.tiles_m, j.tiles_n, j.group, tm, tn);
+  const int il = bx * 4 + ((int)threadIdx.x >> 6), jl = ((int)threadIdx.x & 63) * 4;
   float4 s = {0.f, 0.f, 0.f, 0.f};
-  for (int p = 0; p < P; ++p) {
-    const float4 v = *reinterpret_cast<const float4*>(part + ((int64_t)(r * P + p) * BM + il) * BN + jl);
+  const float* src = j.part + ((int64_t)r * j.P * BM + il) * BN + jl;
+#pragma unroll 4
+  for (int p = 0; p < j.P; ++p) {
+    const float4 v = *reinterpret_cast<const float4*>(src + (int64_t)p * BM * BN);
     s.x += v.x;
     s.y += v.y;
     s.z += v.z;
     s.w += v.w;
   }
   const int64_t i = (int64_t)tm * BM + il;
-  if (i >= M) return;
-  const float gs = go != nullptr ? go[0] : 1.f;
-  const float sc = rscale != nullptr ? gs * rscale[i] : gs;
+  if (i >= j.M) return;
+  const float gs = j.go != nullptr ? j.go[0] : 1.f;
+  const float sc = j.rscale != nullptr ? gs * j.rscale[i] : gs;
   const float o[4] = {s.x, s.y, s.z, s.w};
   float c[4] = {0.f, 0.f, 0.f, 0.f};  // Cin loaded before the stores (it may be C itself)
-  if (!OUT_BF16 && cin != nullptr) {
+  if (!OUT_BF16 && j.cin != nullptr) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int64_t j = (int64_t)tn * BN + jl + e;
-      if (j < Nc) c[e] = cin[i * ldc + j];
+      const int64_t col = (int64_t)tn * BN + jl + e;
+      if (col < j.Nx) c[e] = j.cin[i * j.ldc + col];
     }
   }
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const int64_t j = (int64_t)tn * BN + jl + e;
-    if (j < Nc) {
+    const int64_t col = (int64_t)tn * BN + jl + e;
+    if (col < j.Nx) {
       if constexpr (OUT_BF16)
-        reinterpret_cast<__bf16*>(C)[i * ldc + j] = (__bf16)(sc * o[e]);
+        reinterpret_cast<__bf16*>(j.C)[i * j.ldc + col] = (__bf16)(sc * o[e]);
       else
-        reinterpret_cast<float*>(C)[i * ldc + j] = sc * (o[e] + c[e]);
+        reinterpret_cast<float*>(j.C)[i * j.ldc + col] = sc * (o[e] + c[e]);
     }
   }
 }
 
-// The extra columns (k_gemm's XM) of the K-split tail tiles: block (tail tile r, group j) adds the P slices' values
+// The extra columns (k_gemm's XM) of the K-split tail tiles: (tail tile r, group g) adds the P slices' values
 // of its 32 rows in a fixed order and writes them with k_gemm's epilogue (row scale, go, Cin). Thread t: row i = t/8,
 // extra columns 4(t%8) .. +3.
 template <bool OUT_BF16>
-__global__ __launch_bounds__(256) void k_xtail_reduce(const float* __restrict__ xpart, int P, int full, int nr,
-                                                      int tiles_m, int tiles_n, int group, int am2, int64_t M,
-                                                      int64_t Nx, int xcols, void* C, int64_t ldc,
-                                                      const float* __restrict__ rscale, const float* __restrict__ go,
-                                                      const float* cin) {
-  const int r = (int)blockIdx.x, j = (int)blockIdx.y, t = threadIdx.x;
+__device__ __forceinline__ void xtail_reduce(const TailJob& j, int r, int g) {
+  const int t = threadIdx.x;
   int tm, tn;
-  tile_of(full + r, tiles_m, tiles_n, group, tm, tn);
-  const int rg = tn + j * tiles_n;
+  tile_of(j.full + r, j.tiles_m, j.tiles_n, j.group, tm, tn);
+  const int rg = tn + g * j.tiles_n;
   if (tn >= 8 || rg > 7) return;
   const int i = t >> 3;
-  const int64_t row = (int64_t)tm * BM + rg * 32 + (am2 ? kperm_inv(i) : i);
-  if (row >= M) return;
-  const float gs = go != nullptr ? go[0] : 1.f;
-  const float sc = rscale != nullptr ? gs * rscale[row] : gs;
+  const int64_t row = (int64_t)tm * BM + rg * 32 + (j.am2 ? kperm_inv(i) : i);
+  if (row >= j.M) return;
+  const float gs = j.go != nullptr ? j.go[0] : 1.f;
+  const float sc = j.rscale != nullptr ? gs * j.rscale[row] : gs;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int n = 4 * (t & 7) + q;
-    if (n >= xcols) continue;
+    if (n >= j.xcols) continue;
     float v = 0.f;
-    for (int p = 0; p < P; ++p) v += xpart[((((int64_t)r * P + p) * nr + j) * 32 + i) * 32 + n];
-    const int64_t col = Nx + n;
+    for (int p = 0; p < j.P; ++p) v += j.xpart[((((int64_t)r * j.P + p) * j.nr + g) * 32 + i) * 32 + n];
+    const int64_t col = j.Nx + n;
     if constexpr (OUT_BF16)
-      reinterpret_cast<__bf16*>(C)[row * ldc + col] = (__bf16)(sc * v);
+      reinterpret_cast<__bf16*>(j.C)[row * j.ldc + col] = (__bf16)(sc * v);
     else
-      reinterpret_cast<float*>(C)[row * ldc + col] = sc * (v + (cin != nullptr ? cin[row * ldc + col] : 0.f));
+      reinterpret_cast<float*>(j.C)[row * j.ldc + col] = sc * (v + (j.cin != nullptr ? j.cin[row * j.ldc + col] : 0.f));
   }
+}
+template <bool OUT_BF16>
+__device__ __forceinline__ void tail_block(const TailJob& j, int b) {
+  const int q = b - j.tails * (BM / 4);
+  if (q < 0)
+    tail_reduce<OUT_BF16>(j, b % (BM / 4), b / (BM / 4));
+  else
+    xtail_reduce<OUT_BF16>(j, q % j.tails, q / j.tails);
+}
+template <bool OUT_BF16>
+__global__ __launch_bounds__(256) void k_tail_reduce(TailJob j) {
+  tail_block<OUT_BF16>(j, (int)blockIdx.x);
 }
 
 // dBias of the training path from the dW blocks' dot-product partials (k_gemm<.., DB>): row group rg = (v%256)/32
@@ -2542,22 +2587,69 @@ __device__ __forceinline__ int lin_of(int tm, int tn, int tiles_m, int tiles_n, 
   const int g = tm / group, first = g * group, gsize = min(tiles_m - first, group);
   return g * group * tiles_n + tn * gsize + (tm - first);
 }
-__global__ __launch_bounds__(256) void k_dbias_tiles(const float* __restrict__ upart, int tiles_m, int tiles_n,
-                                                     int nr, int group, int full, int P, int64_t V,
-                                                     const float* __restrict__ go, const float* cin, float* dbias) {
-  const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (v >= V) return;
+struct BiasJob {
+  const float* upart;
+  int tiles_m, tiles_n, nr, group, full, P;
+  int64_t V;
+  const float *go, *cin;
+  float* dbias;
+};
+__device__ __forceinline__ void dbias_tiles(const BiasJob& j, int b) {
+  const int64_t v = (int64_t)b * 256 + threadIdx.x;
+  if (v >= j.V) return;
   const int tm = (int)(v / BM), rg = (int)((v % BM) / 32), m = (int)(v % 32);
-  const int tn = rg % tiles_n, j = rg / tiles_n;
-  const int64_t T = (int64_t)tiles_m * tiles_n;
-  const int lin = lin_of(tm, tn, tiles_m, tiles_n, group);
+  const int tn = rg % j.tiles_n, g = rg / j.tiles_n;
+  const int64_t T = (int64_t)j.tiles_m * j.tiles_n;
+  const int lin = lin_of(tm, tn, j.tiles_m, j.tiles_n, j.group);
   float s = 0.f;
-  if (lin < full) {
-    s = upart[((int64_t)lin * nr + j) * 32 + m];
+  if (lin < j.full) {
+    s = j.upart[((int64_t)lin * j.nr + g) * 32 + m];
   } else {
-    for (int p = 0; p < P; ++p) s += upart[((T + (int64_t)(lin - full) * P + p) * nr + j) * 32 + m];
+    for (int p = 0; p < j.P; ++p) s += j.upart[((T + (int64_t)(lin - j.full) * j.P + p) * j.nr + g) * 32 + m];
   }
-  dbias[v] = (go != nullptr ? go[0] : 1.f) * (s + (cin != nullptr ? cin[v] : 0.f));
+  j.dbias[v] = (j.go != nullptr ? j.go[0] : 1.f) * (s + (j.cin != nullptr ? j.cin[v] : 0.f));
+}
+
+// The small passes between and after the two contractions of a block, several in one launch: a launch of its own costs
+// each of them some 5 us, more than its work at any but the largest sizes.
+// Between: the dH tail tiles (first: they wait for nothing else and take longest), dGate = go * dgr over all N rows,
+// and the scaled H^T copy for dW (transpose_tile on a tr_x x tr_y grid; tr_x = 0: none).
+struct MidJob {
+  TailJob dh;
+  const float *dgr, *dgate_go;
+  float* dgate;
+  int64_t N;
+  const uint16_t* H;
+  int64_t ldh, rows, K;
+  uint16_t* Ht;
+  const float* rscale;
+  uint16_t* uperm;
+  int tr_x, tr_y, gate_blocks;
+};
+template <bool DH_BF16>
+__global__ __launch_bounds__(256) void k_grads_mid(MidJob j) {
+  __shared__ __attribute__((aligned(16))) TransposeTile tile;
+  int b = (int)blockIdx.x;
+  if (b < j.dh.blocks()) {
+    tail_block<DH_BF16>(j.dh, b);
+    return;
+  }
+  b -= j.dh.blocks();
+  if (b < j.gate_blocks) {
+    const int64_t n = (int64_t)b * 256 + threadIdx.x;
+    if (n < j.N) j.dgate[n] = j.dgate_go[0] * j.dgr[n];
+    return;
+  }
+  b -= j.gate_blocks;
+  transpose_tile(j.H, j.ldh, j.rows, j.K, j.Ht, j.rscale, nullptr, j.uperm, 1, tile, b % j.tr_x, b / j.tr_x);
+}
+// After: the dW tail tiles, then dBias.
+__global__ __launch_bounds__(256) void k_grads_end(TailJob dw, BiasJob bias) {
+  const int b = (int)blockIdx.x;
+  if (b < dw.blocks())
+    tail_block<false>(dw, b);
+  else
+    dbias_tiles(bias, b - dw.blocks());
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -2751,14 +2843,14 @@ class ProfScope {
 
 // C = s_i (A . B^T + Cin) over nk stages with the tile grid of k_gemm (s_i, Cin as there). When the tiles leave a
 // partial last wave (or do not fill the GPU once), the R tail tiles are split into P = CUs / R K-slices (at least 2
-// stages each) so the last wave fills the GPU.
+// stages each) so the last wave fills the GPU. The tails' reduction is launched here or, with `tail`, left to the caller
+// (no blocks when nothing was split).
 int launch_status();
 template <bool OUT_BF16>
 int launch_gemm(const Operand& A, const Operand& B, int nk, int64_t M, int64_t Nc, int group, void* C, int64_t ldc,
                 float* part, hipStream_t st, const float* rscale = nullptr, const float* go = nullptr,
                 const float* cin = nullptr, const uint16_t* u = nullptr, float* upart = nullptr,
-                int* p_out = nullptr, int* full_out = nullptr, int pcls = PROF_NONE, const Operand* X = nullptr,
-                float* xpart = nullptr) {
+                int pcls = PROF_NONE, const Operand* X = nullptr, float* xpart = nullptr, TailJob* tail = nullptr) {
   // with X (extra-column mode), the last X->mext (<= 32) of the Nc columns are formed inside the tiles of the others
   const int64_t Nx = X != nullptr ? Nc - X->mext : Nc;
   const int tiles_m = (int)cdiv(M, BM), tiles_n = (int)cdiv(Nx, BN), T = tiles_m * tiles_n;
@@ -2776,8 +2868,6 @@ int launch_gemm(const Operand& A, const Operand& B, int nk, int64_t M, int64_t N
   const bool kf = A.kext % BK == 0 && B.kext % BK == 0;
   const dim3 grid(full + (T - full) * P);
   if (B.cm) return MCE_EINVAL;  // only the A operand may be in the piece layout
-  if (p_out) *p_out = P;
-  if (full_out) *full_out = full;
   // transposed pieces (G read with the vocabulary as M, for dW): whole K stages only. Dot products with u: only
   // with such an A operand and fp32 output. The extra-column mode: whole K stages, 1 or 2 row groups per tile, no u
   const int nr = fold_nr(tiles_n);
@@ -2846,13 +2936,12 @@ int launch_gemm(const Operand& A, const Operand& B, int nk, int64_t M, int64_t N
                          tiles_m, tiles_n, group, full, P, C, ldc, part, rscale, go, cin, nullptr, nullptr, none, Nc);
   }
   prof.end();
-  int rc = launch_status();
-  if (rc || full == T) return rc;
-  hipLaunchKernelGGL((k_tail_reduce<OUT_BF16>), dim3(BM / 4, T - full), dim3(256), 0, st, part, P, full, tiles_m,
-                     tiles_n, group, M, Nx, C, ldc, rscale, go, cin);
-  if ((rc = launch_status()) || X == nullptr) return rc;
-  hipLaunchKernelGGL((k_xtail_reduce<OUT_BF16>), dim3(T - full, nr), dim3(256), 0, st, xpart, P, full, nr, tiles_m,
-                     tiles_n, group, A.cm == 2 ? 1 : 0, M, Nx, (int)X->mext, C, ldc, rscale, go, cin);
+  const int rc = launch_status();
+  const TailJob job{part, xpart, P, full, T - full, nr, tiles_m, tiles_n, group, A.cm == 2 ? 1 : 0,
+                    X != nullptr ? (int)X->mext : 0, M, Nx, C, ldc, rscale, go, cin};
+  if (tail != nullptr) *tail = job;
+  if (rc || full == T || tail != nullptr) return rc;
+  hipLaunchKernelGGL((k_tail_reduce<OUT_BF16>), dim3((unsigned)job.blocks()), dim3(256), 0, st, job);
   return launch_status();
 }
 
@@ -2922,8 +3011,8 @@ int fwd_launch(const FwdWs& w, const uint16_t* H, int64_t ldh, const uint16_t* W
   }
   if ((rc = launch_status())) return rc;
   hipLaunchKernelGGL(k_fwd_merge, dim3((unsigned)cdiv(N, 32)), dim3(256), 0, st, w.part_m, w.part_s, xy, w.cb, w.xc,
-                     kc, gate, hit, N, 2 * tv, loss_rows, lse_rows, wgt_rows, dgr_rows, nullptr,
-                     kc > 0 ? w.xcount : nullptr, w.xlist);
+                     kc, gate, hit, N, 2 * tv, loss_rows, lse_rows, wgt_rows, dgr_rows, kc > 0 ? w.xcount : nullptr, w.xlist,
+                     TrainRows{});
   if ((rc = launch_status())) return rc;
   if (kc == 0) return MCE_OK;
   return launch_exact(H, ldh, W, ldw, bias, cand, cval, kc, N, K, V, V_real, tv, w.xcount, w.xlist, w.part_m,
@@ -3065,9 +3154,9 @@ int block_contractions(const BwdWs& w, const uint16_t* H, int64_t ldh, int64_t N
     const Operand Xop{w.Wt + (K - kx) * BLK, BLK, kx, w.vp, K * BLK};
     const int nk = (int)(w.vp / BK);
     rc = dh_bf16 ? launch_gemm<true>(Aop, Bop, nk, N, K, 4, dH, lddh, w.part, st, nullptr, nullptr, nullptr, nullptr,
-                                     nullptr, nullptr, nullptr, PROF_GEMM_DH, kx ? &Xop : nullptr, w.xpart)
+                                     nullptr, PROF_GEMM_DH, kx ? &Xop : nullptr, w.xpart)
                  : launch_gemm<false>(Aop, Bop, nk, N, K, 4, dH, lddh, w.part, st, nullptr, nullptr, nullptr, nullptr,
-                                      nullptr, nullptr, nullptr, PROF_GEMM_DH, kx ? &Xop : nullptr, w.xpart);
+                                      nullptr, PROF_GEMM_DH, kx ? &Xop : nullptr, w.xpart);
     if (rc) return rc;
   }
   if (dW == nullptr) return MCE_OK;
@@ -3078,7 +3167,7 @@ int block_contractions(const BwdWs& w, const uint16_t* H, int64_t ldh, int64_t N
   const Operand Bop{w.Ht, BLK, K, np, K * BLK, 0};
   const Operand Xop{w.Ht + (K - kx) * BLK, BLK, kx, np, K * BLK, 0};
   return launch_gemm<false>(Aop, Bop, (int)(np / BK), V, K, 4, dW, lddw, w.part, st, nullptr, nullptr, dW_in, nullptr,
-                            nullptr, nullptr, nullptr, PROF_GEMM_DW, kx ? &Xop : nullptr, w.xpart);
+                            nullptr, PROF_GEMM_DW, kx ? &Xop : nullptr, w.xpart);
 }
 
 // The whole recompute backward of every variant, block by block: per block the logits gradient (grad_launch),
@@ -3210,44 +3299,74 @@ thread_local float t_train_s_max = TRAIN_S_MAX;  // test hook: mce_train_set_thr
 // be null; dW_in / dBias_in may be null (none) or equal to the outputs (an accumulation).
 int train_block_grads(const TrainWs& w, int64_t b, const uint16_t* H, int64_t ldh, int64_t N, int64_t K,
                       int64_t V, const float* go, void* dH, int dh_bf16, int64_t lddh, float* dW, int64_t lddw,
-                      const float* dW_in, float* dBias, const float* dBias_in, hipStream_t st) {
+                      const float* dW_in, float* dBias, const float* dBias_in, float* dGate, const float* dgr,
+                      hipStream_t st) {
   int rc;
   const int64_t row0 = b * w.nb, rows = std::min(w.nb, N - row0), rp = cdiv(rows, BLK) * BLK;
   const int64_t kx = extra_cols(K);
+  MidJob mid{};
   if (dH != nullptr) {
     const Operand Aop{w.G, 0, rows, w.vp, rp * BLK, 1};
     const Operand Bop{w.Wt, BLK, K, w.vp, K * BLK};
     const Operand Xop{w.Wt + (K - kx) * BLK, BLK, kx, w.vp, K * BLK};   // W^T's last kx rows
     const int nk = (int)(w.vp / BK);
     rc = dh_bf16 ? launch_gemm<true>(Aop, Bop, nk, rows, K, 4, reinterpret_cast<uint16_t*>(dH) + row0 * lddh, lddh,
-                                     w.part, st, w.arow + row0, go, nullptr, nullptr, nullptr, nullptr, nullptr,
-                                     PROF_GEMM_DH, kx ? &Xop : nullptr, w.xpart)
+                                     w.part, st, w.arow + row0, go, nullptr, nullptr, nullptr, PROF_GEMM_DH,
+                                     kx ? &Xop : nullptr, w.xpart, &mid.dh)
                  : launch_gemm<false>(Aop, Bop, nk, rows, K, 4, reinterpret_cast<float*>(dH) + row0 * lddh, lddh,
-                                      w.part, st, w.arow + row0, go, nullptr, nullptr, nullptr, nullptr, nullptr,
-                                      PROF_GEMM_DH, kx ? &Xop : nullptr, w.xpart);
+                                      w.part, st, w.arow + row0, go, nullptr, nullptr, nullptr, PROF_GEMM_DH,
+                                      kx ? &Xop : nullptr, w.xpart, &mid.dh);
     if (rc) return rc;
+  }
+  if (dGate != nullptr) {
+    mid.dgr = dgr;
+    mid.dgate_go = go;
+    mid.dgate = dGate;
+    mid.N = N;
+    mid.gate_blocks = (int)cdiv(N, 256);
+  }
+  if (dW != nullptr) {
+    // H^T of the block scaled by a (and, for dBias, a itself in bf16); dW = E'^T (a . H), and the dW tiles also form
+    // the dBias partials sum_n E'[n, v] a_n, each over its share of the K stages (dbias_tiles adds them)
+    mid.H = H + row0 * ldh;
+    mid.ldh = ldh;
+    mid.rows = rows;
+    mid.K = K;
+    mid.Ht = w.Ht;
+    mid.rscale = w.arow + row0;
+    mid.uperm = dBias ? w.uperm : nullptr;
+    mid.tr_x = (int)(rp / 64);
+    mid.tr_y = (int)cdiv(K, 64);
+  }
+  const int64_t mid_blocks = mid.dh.blocks() + mid.gate_blocks + (int64_t)mid.tr_x * mid.tr_y;
+  if (mid_blocks > 0) {
+    if (dh_bf16)
+      hipLaunchKernelGGL(k_grads_mid<true>, dim3((unsigned)mid_blocks), dim3(256), 0, st, mid);
+    else
+      hipLaunchKernelGGL(k_grads_mid<false>, dim3((unsigned)mid_blocks), dim3(256), 0, st, mid);
+    if ((rc = launch_status())) return rc;
   }
   if (dW == nullptr && dBias == nullptr) return MCE_OK;
   if (dW != nullptr) {
-    // H^T of the block scaled by a (and, for dBias, a itself in bf16); dW = E'^T (a . H), and the dW tiles also form
-    // the dBias partials sum_n E'[n, v] a_n, each over its share of the K stages (k_dbias_tiles adds them)
-    hipLaunchKernelGGL(k_transpose_blocked, dim3((unsigned)(rp / 64), (unsigned)cdiv(K, 64)), dim3(256), 0, st,
-                       H + row0 * ldh, ldh, rows, K, w.Ht, w.arow + row0, nullptr, dBias ? w.uperm : nullptr, 1);
-    if ((rc = launch_status())) return rc;
     // G read transposed: M = the vocabulary (v tiles rp*256 elements apart), K = the block's rows (row tiles
-    // 65536 elements apart)
-    const Operand Aop{w.G, rp * BLK, V, rp, CM_TILE, 2};
-    const Operand Bop{w.Ht, BLK, K, rp, K * BLK, 0};
-    const Operand Xop{w.Ht + (K - kx) * BLK, BLK, kx, rp, K * BLK, 0};   // (a . H)^T's last kx rows
+    // 65536 elements apart), whole stages up to the last row (the rows past it up to rp are zero in both operands)
+    const int64_t rk = cdiv(rows, BK) * BK;
+    const Operand Aop{w.G, rp * BLK, V, rk, CM_TILE, 2};
+    const Operand Bop{w.Ht, BLK, K, rk, K * BLK, 0};
+    const Operand Xop{w.Ht + (K - kx) * BLK, BLK, kx, rk, K * BLK, 0};   // (a . H)^T's last kx rows
     const bool xm = kx > 0 && dBias == nullptr;   // the dBias dot products take the extra-column slot otherwise
-    int P = 1, full = 0;
-    if ((rc = launch_gemm<false>(Aop, Bop, (int)(rp / BK), V, K, 4, dW, lddw, w.part, st, nullptr, go, dW_in,
-                                 dBias ? w.uperm : nullptr, w.upart, &P, &full, PROF_GEMM_DW, xm ? &Xop : nullptr,
-                                 w.xpart)))
+    TailJob tail{};
+    if ((rc = launch_gemm<false>(Aop, Bop, (int)(rk / BK), V, K, 4, dW, lddw, w.part, st, nullptr, go, dW_in,
+                                 dBias ? w.uperm : nullptr, w.upart, PROF_GEMM_DW, xm ? &Xop : nullptr, w.xpart,
+                                 &tail)))
       return rc;
-    if (dBias == nullptr) return MCE_OK;
-    hipLaunchKernelGGL(k_dbias_tiles, dim3((unsigned)cdiv(V, 256)), dim3(256), 0, st, w.upart, (int)cdiv(V, BM),
-                       (int)cdiv(K, BN), fold_nr(cdiv(K, BN)), 4, full, P, V, go, dBias_in, dBias);
+    BiasJob bias{};
+    if (dBias != nullptr)
+      bias = BiasJob{w.upart, (int)cdiv(V, BM), (int)cdiv(K, BN), fold_nr(cdiv(K, BN)), 4, tail.full, tail.P, V, go,
+                     dBias_in, dBias};
+    const int64_t blocks = tail.blocks() + (dBias != nullptr ? cdiv(V, 256) : 0);
+    if (blocks == 0) return MCE_OK;
+    hipLaunchKernelGGL(k_grads_end, dim3((unsigned)blocks), dim3(256), 0, st, tail, bias);
     return launch_status();
   }
   // dBias without dW: a pass over the block's G
@@ -3327,39 +3446,41 @@ int fwd_train_impl(const uint16_t* H, int64_t ldh, uint16_t* W, int64_t ldw, con
     }
     if ((rc = launch_status())) return rc;
     int* xcount = w.counts + w.np / BLK + b;
-    hipLaunchKernelGGL(k_fwd_merge, dim3((unsigned)cdiv(rows, 32)), dim3(256), 0, st, w.part_m, w.part_s,
-                       w.xy + row0, w.cb + row0 * kc, w.xc + row0 * kc, kc, at(gate, row0), at(hit, row0), rows, 2 * tv, loss_rows + row0, lse_rows + row0,
-                       wgt_rows + row0, at(dgr_rows, row0), nullptr, kc > 0 ? xcount : nullptr, w.xlist);
+    const TrainRows tr{y + row0, w.lse_est + row0, w.flag + row0, rp, V_real, w.arow + row0, w.counts + b, w.flag_list,
+                       w.G};
+    hipLaunchKernelGGL(k_fwd_merge, dim3((unsigned)(rp / 32)), dim3(256), 0, st, w.part_m, w.part_s, w.xy + row0,
+                       w.cb + row0 * kc, w.xc + row0 * kc, kc, at(gate, row0), at(hit, row0), rows, 2 * tv,
+                       loss_rows + row0, lse_rows + row0, wgt_rows + row0, at(dgr_rows, row0),
+                       kc > 0 ? xcount : nullptr, w.xlist, kc > 0 ? TrainRows{} : tr);
     if ((rc = launch_status())) return rc;
-    if (kc > 0 && (rc = launch_exact(H + row0 * ldh, ldh, W, ldw, bias, at(cand, row0 * kc), at(cval, row0 * kc), kc,
-                                     rows, K, V, V_real, tv, xcount, w.xlist, w.part_m, w.part_s, w.xy + row0,
-                                     loss_rows + row0, lse_rows + row0, wgt_rows + row0, st)))
-      return rc;
-    hipLaunchKernelGGL(k_train_rows, dim3((unsigned)(rp / 256)), dim3(256), 0, st, y + row0, w.xy + row0,
-                       at(cand, row0 * kc), w.cb + row0 * kc, w.xc + row0 * kc, kc, w.lse_est + row0,
-                       lse_rows + row0, wgt_rows + row0, w.flag + row0, rows, rp, V_real, w.arow + row0,
-                       w.counts + b, w.flag_list, w.G);
-    if ((rc = launch_status())) return rc;
+    if (kc > 0) {
+      if ((rc = launch_exact(H + row0 * ldh, ldh, W, ldw, bias, at(cand, row0 * kc), at(cval, row0 * kc), kc, rows, K,
+                             V, V_real, tv, xcount, w.xlist, w.part_m, w.part_s, w.xy + row0, loss_rows + row0,
+                             lse_rows + row0, wgt_rows + row0, st)))
+        return rc;
+      hipLaunchKernelGGL(k_train_rows, dim3((unsigned)(rp / 256)), dim3(256), 0, st, tr, at(cand, row0 * kc),
+                         w.cb + row0 * kc, w.xc + row0 * kc, kc, w.xy + row0, lse_rows + row0, wgt_rows + row0, rows);
+      if ((rc = launch_status())) return rc;
+    }
     // the flagged rows' exact E' (the block's H^T buffer, rewritten later, holds their gathered rows)
-    hipLaunchKernelGGL(k_gather_rows, dim3(REPAIR_BLOCKS), dim3(256), 0, st, H + row0 * ldh, ldh, w.flag_list,
-                       w.counts + b, K, w.Ht);
+    const bool sums = b + 1 == w.nblk && N <= SUM_ONE_BLOCK;   // every row's loss is final: its last writer has run
+    hipLaunchKernelGGL(k_gather_rows, dim3(REPAIR_BLOCKS / 4 + 1), dim3(1024), 0, st, H + row0 * ldh, ldh, w.flag_list,
+                       w.counts + b, K, w.Ht, loss_rows, N, sums ? loss_sum : nullptr);
     if ((rc = launch_status())) return rc;
     MCE_LAUNCH_KM(k_exact_train, K, dim3((unsigned)(tv * tnb)), dim3(NTHREADS), 0, st, Wop, w.Ht, K, bias, w.counts + b,
-                  w.flag_list, lse_rows + row0, rp, V, V_real, tv, w.G);
-    if ((rc = launch_status())) return rc;
-    hipLaunchKernelGGL(k_exact_fix, dim3((unsigned)(rp / 256)), dim3(256), 0, st, w.counts + b, w.flag_list, y + row0,
-                       w.xy + row0, at(cand, row0 * kc), w.cb + row0 * kc, w.xc + row0 * kc, kc, lse_rows + row0,
-                       rp, V_real, w.G);
+                  w.flag_list, lse_rows + row0, rp, V, V_real, tv, w.G,
+                  ExactFix{y + row0, at(cand, row0 * kc), w.xy + row0, w.cb + row0 * kc, w.xc + row0 * kc, kc});
     if ((rc = launch_status())) return rc;
     if (b + 1 < w.nblk) {
       const bool first = b == 0;
       if ((rc = train_block_grads(w, b, H, ldh, N, K, V, nullptr, (want & MCE_GRAD_H) ? dH_part : nullptr, dh_bf16,
                                   lddh, (want & MCE_GRAD_W) ? dW_part : nullptr, lddw, first ? nullptr : dW_part,
-                                  (want & MCE_GRAD_BIAS) ? dBias_part : nullptr, first ? nullptr : dBias_part, st)))
+                                  (want & MCE_GRAD_BIAS) ? dBias_part : nullptr, first ? nullptr : dBias_part, nullptr,
+                                  nullptr, st)))
         return rc;
     }
   }
-  return launch_sum(loss_rows, N, w.sum_part, loss_sum, st);
+  return N <= SUM_ONE_BLOCK ? MCE_OK : launch_sum(loss_rows, N, w.sum_part, loss_sum, st);
 }
 
 // Backward of the one-pass training path: the last block's contractions with go, added to the partial sums of the
@@ -3383,7 +3504,7 @@ int bwd_train_impl(const uint16_t* H, int64_t ldh, const float* go, const float*
     if (dBias) hipLaunchKernelGGL(k_fill_f32, dim3((unsigned)cdiv(V, 256)), dim3(256), 0, st, dBias, V, 0.f);
     return launch_status();
   }
-  if (!ws) return MCE_EINVAL;
+  if (!ws || (dGate && !dgr_rows)) return MCE_EINVAL;
   const TrainWs w = train_ws_layout(reinterpret_cast<char*>(ws), N, K, V, block_rows);
   if (ws_bytes < w.bytes) return MCE_EWORKSPACE;
   const int64_t b = w.nblk - 1, row0 = b * w.nb;
@@ -3398,15 +3519,8 @@ int bwd_train_impl(const uint16_t* H, int64_t ldh, const float* go, const float*
                          lddh, row0, K, go);
     if ((rc = launch_status())) return rc;
   }
-  if ((rc = train_block_grads(w, b, H, ldh, N, K, V, go, dH, dh_bf16, lddh, dW, lddw, row0 > 0 ? dW_part : nullptr,
-                              dBias, row0 > 0 ? dBias_part : nullptr, st)))
-    return rc;
-  if (dGate) {
-    if (!dgr_rows) return MCE_EINVAL;
-    hipLaunchKernelGGL(k_dgate, dim3((unsigned)cdiv(N, 256)), dim3(256), 0, st, dgr_rows, go, N, dGate);
-    return launch_status();
-  }
-  return MCE_OK;
+  return train_block_grads(w, b, H, ldh, N, K, V, go, dH, dh_bf16, lddh, dW, lddw, row0 > 0 ? dW_part : nullptr, dBias,
+                           row0 > 0 ? dBias_part : nullptr, dGate, dgr_rows, st);
 }
 
 // chunk_ce's backward on the one-pass path: after mce_fwd_train (plain cross-entropy, one row block) the workspace
@@ -3440,7 +3554,8 @@ int bwd_lse_train_impl(const uint16_t* H, int64_t ldh, const int64_t* y, const f
   hipLaunchKernelGGL(k_onehot_rows, dim3((unsigned)(w.vp / BM), 8), dim3(256), 0, st, w.ocount, w.olist, y, w.np,
                      w.G);
   if ((rc = launch_status())) return rc;
-  return train_block_grads(w, 0, H, ldh, N, K, V, nullptr, dH, dh_bf16, lddh, dW, lddw, nullptr, dBias, nullptr, st);
+  return train_block_grads(w, 0, H, ldh, N, K, V, nullptr, dH, dh_bf16, lddh, dW, lddw, nullptr, dBias, nullptr,
+                           nullptr, nullptr, st);
 }
 
 }  // namespace
@@ -3605,9 +3720,9 @@ int mce_bwd_dhidden(const uint16_t* W, int64_t ldw, int64_t N, int64_t K, int64_
   const Operand Bop{w.Wt, BLK, K, w.vp, K * BLK};
   const int nk = (int)(w.vp / BK);
   return dh_bf16 ? launch_gemm<true>(Aop, Bop, nk, N, K, 4, dH, lddh, w.part, st, nullptr, nullptr, nullptr, nullptr,
-                                     nullptr, nullptr, nullptr, PROF_GEMM_DH)
+                                     nullptr, PROF_GEMM_DH)
                  : launch_gemm<false>(Aop, Bop, nk, N, K, 4, dH, lddh, w.part, st, nullptr, nullptr, nullptr, nullptr,
-                                      nullptr, nullptr, nullptr, PROF_GEMM_DH);
+                                      nullptr, PROF_GEMM_DH);
 }
 
 int mce_bwd_dweight(const uint16_t* H, int64_t ldh, int64_t N, int64_t K, int64_t V, float* dW, int64_t lddw,
@@ -3632,7 +3747,7 @@ int mce_bwd_dweight(const uint16_t* H, int64_t ldh, int64_t N, int64_t K, int64_
   const Operand Aop{w.G, w.np * BLK, V, w.np, CM_TILE, 2};
   const Operand Bop{w.Ht, BLK, K, w.np, K * BLK, 0};
   return launch_gemm<false>(Aop, Bop, (int)(w.np / BK), V, K, 4, dW, lddw, w.part, st, nullptr, nullptr, nullptr,
-                            nullptr, nullptr, nullptr, nullptr, PROF_GEMM_DW);
+                            nullptr, nullptr, PROF_GEMM_DW);
 }
 
 int mce_bwd(const uint16_t* H, int64_t ldh, const uint16_t* W, int64_t ldw, const float* bias, const int64_t* y,

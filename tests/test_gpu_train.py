@@ -51,6 +51,21 @@ def test_capi_parity(shape):
     assert_parity(got, dict(fwd, loss_sum=fwd["loss_sum"] * go), bwd, f"train {shape}")
 
 
+@pytest.mark.parametrize("block_rows", [0, 256], ids=["one_block", "blocks256"])
+@pytest.mark.parametrize("N", [1, 63, 64, 65, 128, 129, 255, 257, 321, 577])
+@pytest.mark.parametrize("K,bias", [(264, True), (1040, False), (512, False)])
+def test_reduction_stages_of_partial_row_tiles(K, bias, N, block_rows):
+    """dW reduces over whole 64-row stages up to a block's last row, not up to its padded 256 rows: one stage (64 rows
+    or fewer), stage edges, and row blocks that end a row past one; with the dBias dot products, the extra columns, and
+    neither."""
+    print(f"case N={N} K={K} bias={bias} block_rows={block_rows}", flush=True)
+    case = random_case(N, K, 900, 890 if bias else None, bias, seed=N + K)
+    go = 1.0 / N
+    got = capi_train(case, go=go, block_rows=block_rows)
+    fwd, bwd = oracle_of(case, go=go)
+    assert_parity(got, dict(fwd, loss_sum=fwd["loss_sum"] * go), bwd, f"stages {N} {K}")
+
+
 BLOCK_SHAPES = [
     # several 256-row blocks, the last one ragged: (N, K, V, v_real, bias)
     (777, 520, 2051, 2000, True),      # 4 blocks (256, 256, 256, 9 rows)
@@ -362,7 +377,7 @@ EXTRA_COL_SHAPES = [
 @pytest.mark.parametrize("shape", EXTRA_COL_SHAPES, ids=lambda s: "N{}_K{}_V{}_vr{}_b{}".format(*s))
 def test_extra_columns_inside_the_tiles(shape, path, monkeypatch):
     """Widths K = 256 c + x (0 < x <= 32, c >= 4): dH's and dW's last x columns come from one extra MFMA per row
-    group and stage inside the other tiles (and from k_xtail_reduce for K-split tail tiles), on the one-pass and
+    group and stage inside the other tiles (and from xtail_reduce for K-split tail tiles), on the one-pass and
     recompute paths, in one block and in 256-row blocks, with bf16 and fp32 h."""
     from memarch_amd import fused_ops
     monkeypatch.setattr(fused_ops, "RECOMPUTE", path.startswith("recompute"))
