@@ -1003,6 +1003,135 @@ void k_fwd_tiles(Operand Wop, Operand Hop, const float* __restrict__ bias, int64
   }
 }
 
+// The statistics tiles for at most NARROW_ROWS rows n: 128 vocabulary rows x 64 rows n per workgroup, 32 x 64 per wave.
+// With so few rows the pass is a stream of W, and a 256 x 256 tile spends its time on MFMAs of empty columns (and V/256
+// workgroups leave CUs idle): 64 x 2048 x 50304 takes 48 us against 57 (W alone at the copy rate: 40). K is
+// streamed 64 at a time through three LDS stages of 24 KiB, so that two workgroups of a CU keep up to 144 KiB of loads
+// in flight. Any K; the partials are k_fwd_tiles' (row block = workgroup).
+constexpr int NARROW_ROWS = 64;
+constexpr int NR_V = 128, NR_S = 3, NR_A = NR_V * 128, NR_B = NARROW_ROWS * 128, NR_STAGE = NR_A + NR_B;
+constexpr int NR_LA = NR_A / 4096, NR_LB = NR_B / 4096;  // load instructions per wave and stage
+__global__ __attribute__((amdgpu_flat_work_group_size(NTHREADS, NTHREADS), amdgpu_waves_per_eu(2, 2)))
+void k_fwd_narrow(Operand Wop, Operand Hop, const float* __restrict__ bias, int64_t N, int64_t V, int64_t Vreal,
+                  float* __restrict__ part_m, float* __restrict__ part_s, TargetArgs ta) {
+  __shared__ __attribute__((aligned(1024))) char lds[NR_S * NR_STAGE];
+  __shared__ float bslot[NR_V], red[2][4][NARROW_ROWS];
+  const int t = threadIdx.x, lane = t & 63, lr = lane & 31, lh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int64_t v0 = (int64_t)blockIdx.x * NR_V;
+  const int nk = (int)((Wop.kext + BK - 1) / BK);
+  // instruction j < NR_LA: rows 8 (wave*NR_LA + j) .. +7 of W, else of H; lane l: row l/8, 16-byte chunk (l%8) ^ swz(row)
+  int voff[NR_LA + NR_LB], kloc[NR_LA + NR_LB];
+#pragma unroll
+  for (int j = 0; j < NR_LA + NR_LB; ++j) {
+    const bool b = j >= NR_LA;
+    const int row = (b ? wave * NR_LB + j - NR_LA : wave * NR_LA + j) * 8 + (lane >> 3);
+    const int c = (lane & 7) ^ I::swz(row);
+    const bool in = b ? row < N : v0 + row < V;
+    voff[j] = (int)(row * (b ? Hop.ld : Wop.ld) * 2) + c * 16;
+    kloc[j] = in ? c * 8 : OOB;
+  }
+  auto issue = [&](int stage, int buf) {
+    const int64_t k0 = (int64_t)stage * BK;
+    i32x4 ra = make_rsrc(reinterpret_cast<uint64_t>(Wop.p + v0 * Wop.ld + k0));
+    i32x4 rb = make_rsrc(reinterpret_cast<uint64_t>(Hop.p + k0));
+    const int64_t rest = Wop.kext - k0;
+    const int klim = stage >= nk ? 0 : rest > BK ? BK : (int)rest;
+    if (stage >= nk) ra[2] = rb[2] = 0;
+#pragma unroll
+    for (int j = 0; j < NR_LA + NR_LB; ++j) {
+      const bool b = j >= NR_LA;
+      const int dst = buf * NR_STAGE + (b ? NR_A + (wave * NR_LB + j - NR_LA) * 1024 : (wave * NR_LA + j) * 1024);
+      dma16(b ? rb : ra, lds, dst, kloc[j] < klim ? voff[j] : OOB);
+    }
+  };
+  float bt = 0.f;
+  if (t < NR_V && bias != nullptr) bt = bias[v0 + t < V ? v0 + t : V - 1];
+  int64_t yv[2];
+#pragma unroll
+  for (int nj = 0; nj < 2; ++nj) {
+    yv[nj] = -1;
+    if (ta.xy != nullptr && nj * 32 + lr < N) yv[nj] = ta.y[nj * 32 + lr];
+  }
+#pragma unroll
+  for (int i = 0; i < NR_S; ++i) issue(i, i);
+  f32x16 acc[2];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.f;
+  int buf = 0, kt = 0;
+  const int ra = wave * 32 + lr;
+  do {
+    wait_vmcnt<2 * (NR_LA + NR_LB)>();  // this wave's loads of stage kt; the two later stages' stay in flight
+    __syncthreads();
+    const char* st = lds + buf * NR_STAGE;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      const int c = kk * 2 + lh;
+      const bf16x8 a = frag_at<0>(st, ra * 128 + ((c ^ I::swz(ra)) << 4));
+#pragma unroll
+      for (int nj = 0; nj < 2; ++nj) {
+        const int rb = nj * 32 + lr;
+        acc[nj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            a, frag_at<0>(st, NR_A + rb * 128 + ((c ^ I::swz(rb)) << 4)), acc[nj], 0, 0, 0);
+      }
+    }
+    __syncthreads();  // every wave has read the stage
+    issue(kt + NR_S, buf);
+    buf = buf == NR_S - 1 ? 0 : buf + 1;
+  } while (++kt < nk);
+  wait_vmcnt<0>();  // the loads past the last stage (zeros) land before the workgroup's LDS is given back
+  // the bias and the mask (the bias is loaded ahead of the stages and first used here: a use before the loop would wait
+  // for their loads too, which the compiler does not see)
+  if (t < NR_V) bslot[t] = v0 + t < Vreal ? bt : -INFINITY;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const float b = bslot[wave * 32 + acc_row(0, r, lh)];
+    acc[0][r] += b;
+    acc[1][r] += b;
+  }
+  // the lane holding a row's target writes its logit (plus the row's sparse bias on it, as target_pass)
+#pragma unroll
+  for (int nj = 0; nj < 2; ++nj) {
+    const int64_t d = yv[nj] - (v0 + wave * 32) - 4 * lh;
+    if (yv[nj] >= 0 && yv[nj] < Vreal && d >= 0 && d < 32 && (d & 4) == 0) {
+      float x = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) x = acc_row(0, r, 0) == (int)d ? acc[nj][r] : x;
+      const int64_t n = nj * 32 + lr;
+      for (int k = 0; k < ta.kc; ++k)
+        if (ta.cand[n * ta.kc + k] == yv[nj]) x += ta.cval[n * ta.kc + k];
+      ta.xy[n] = x;
+    }
+    float m = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) m = fmaxf(m, acc[nj][r]);
+    m = fmaxf(m, __shfl_xor(m, 32));
+    float s = 0.f;
+    if (m != -INFINITY) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s += __builtin_amdgcn_exp2f(__builtin_fmaf(acc[nj][r], LOG2E, -m * LOG2E));
+    }
+    s += __shfl_xor(s, 32);
+    if (lh == 0) {
+      red[0][wave][nj * 32 + lr] = m;
+      red[1][wave][nj * 32 + lr] = s;
+    }
+  }
+  __syncthreads();
+  if (t < N && t < NARROW_ROWS) {
+    float m = -INFINITY, s = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) m = fmaxf(m, red[0][w][t]);
+    if (m != -INFINITY) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) s += red[1][w][t] * __builtin_amdgcn_exp2f((red[0][w][t] - m) * LOG2E);
+    }
+    part_m[(int64_t)blockIdx.x * N + t] = m;
+    part_s[(int64_t)blockIdx.x * N + t] = s;
+  }
+}
+
 // Sparse additive logit bias (`linear_ce_sparse`, fused_ops.py:66-101; the eager form full2.py:1920-1922): row
 // n adds cval[n, k] to the logit of vocabulary id cand[n, k] for k < kc. Repeated ids add up (scatter_add);
 // ids outside [0, V_real) are ignored.
@@ -1208,17 +1337,27 @@ __device__ __forceinline__ bool train_row(const TrainRows& tr, int64_t n, float 
 // negative biases remove nearly all of the sum (a candidate that dominates its row pushed far down), the two would
 // cancel each other and leave rounding noise, so a row whose corrected sum is not above 1/16 of the terms removed is
 // appended to exact_list (its lse, loss and wgt are then rewritten by k_exact_tiles / k_exact_rows).
-__global__ __launch_bounds__(256) void k_fwd_merge(const float* __restrict__ part_m, const float* __restrict__ part_s,
-                                                   const float* __restrict__ xy, const float* __restrict__ cb,
+// RB rows per block of NT threads, NT / RB threads per row: 32 rows of 256 threads, or, for at most NARROW_ROWS rows, one
+// block of 64 rows and 1024 threads, which leaves each thread a quarter of the folds (a chain of loads and exponentials
+// that is all of such a merge) and can add up the losses itself (loss_sum not null), in a fixed order. (A count of
+// finished blocks would let any number of blocks do so, but its fence writes back the L2 in every block: 60 us instead
+// of 12 for 4096 rows.)
+// y not null (the statistics pass without sparse candidates, which forms no row logits): xy holds the targets' logits
+// written by the tiles; a target outside [0, Vreal) gets xy = -inf here.
+template <int RB, int NT>
+__global__ __launch_bounds__(NT) void k_fwd_merge(const float* __restrict__ part_m, const float* __restrict__ part_s,
+                                                   float* xy, const float* __restrict__ cb,
                                                    const float* __restrict__ xc, int kc, const float* __restrict__ gate,
                                                    const float* __restrict__ hit, int64_t N, int T,
                                                    float* __restrict__ loss_rows, float* __restrict__ lse_rows,
                                                    float* __restrict__ wgt_rows, float* __restrict__ dgr_rows,
                                                    int* __restrict__ exact_count, int* __restrict__ exact_list,
-                                                   TrainRows tr) {
-  __shared__ float rm[8][32], rs[8][32];
-  const int t = threadIdx.x, r = t & 31, sl = t >> 5;
-  const int64_t n = (int64_t)blockIdx.x * 32 + r;
+                                                   TrainRows tr, const int64_t* __restrict__ y, int64_t Vreal,
+                                                   float* __restrict__ loss_sum) {
+  constexpr int SL = NT / RB;
+  __shared__ float rm[SL][RB], rs[SL][RB];
+  const int t = threadIdx.x, r = t % RB, sl = t / RB;
+  const int64_t n = (int64_t)blockIdx.x * RB + r;
   float m = -INFINITY, s = 0.f;
   if (n < N) {
     int tb = sl;
@@ -1234,54 +1373,50 @@ __global__ __launch_bounds__(256) void k_fwd_merge(const float* __restrict__ par
       m = M4;
     };
     // two folds' loads issued together (16 per thread in flight), folded in the same order as one at a time
-    for (; tb + 56 < T; tb += 64) {
+    for (; tb + 7 * SL < T; tb += 8 * SL) {
       float mm[2][4], ss[2][4];
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          mm[h][q] = part_m[(int64_t)(tb + 32 * h + 8 * q) * N + n];
-          ss[h][q] = part_s[(int64_t)(tb + 32 * h + 8 * q) * N + n];
+          mm[h][q] = part_m[(int64_t)(tb + SL * (4 * h + q)) * N + n];
+          ss[h][q] = part_s[(int64_t)(tb + SL * (4 * h + q)) * N + n];
         }
       fold4(mm[0], ss[0]);
       fold4(mm[1], ss[1]);
     }
-    for (; tb + 24 < T; tb += 32) {
+    for (; tb < T; tb += 4 * SL) {  // the rest: partials past the last count as empty
       float mm[4], ss[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        mm[q] = part_m[(int64_t)(tb + 8 * q) * N + n];
-        ss[q] = part_s[(int64_t)(tb + 8 * q) * N + n];
+        const bool in = tb + SL * q < T;
+        mm[q] = in ? part_m[(int64_t)(tb + SL * q) * N + n] : -INFINITY;
+        ss[q] = in ? part_s[(int64_t)(tb + SL * q) * N + n] : 0.f;
       }
       fold4(mm, ss);
-    }
-    for (; tb < T; tb += 8) {
-      const float mm = part_m[(int64_t)tb * N + n];
-      if (mm == -INFINITY) continue;
-      const float ss = part_s[(int64_t)tb * N + n];
-      if (mm > m) {
-        s = (m == -INFINITY ? 0.f : s * expf(m - mm)) + ss;
-        m = mm;
-      } else {
-        s += ss * expf(mm - m);
-      }
     }
   }
   rm[sl][r] = m;
   rs[sl][r] = s;
   __syncthreads();
   if (sl == 0) {
+    float loss = 0.f;
     if (n >= N) {
       if (tr.G != nullptr && n < tr.Np) tr.arow[n] = 0.f;
     } else {
-      float loss = 0.f, wgt = 0.f;
+      float wgt = 0.f;
       float M = -INFINITY;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) M = fmaxf(M, rm[i][r]);
+      for (int i = 0; i < SL; ++i) M = fmaxf(M, rm[i][r]);
       float S = 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+      for (int i = 0; i < SL; ++i)
         if (rm[i][r] != -INFINITY) S += rs[i][r] * expf(rm[i][r] - M);
+      float xt = -INFINITY;  // the target's logit
+      if (y == nullptr || (y[n] >= 0 && y[n] < Vreal))
+        xt = xy[n];
+      else
+        xy[n] = xt;
       if (kc > 0) {
         float Mp = M;
         for (int k = 0; k < kc; ++k)
@@ -1302,11 +1437,11 @@ __global__ __launch_bounds__(256) void k_fwd_merge(const float* __restrict__ par
       lse_rows[n] = M + ls;
       // lse - x_y as (M - x_y) + log S: M - x_y is exact where x_y is near M, so a row whose p_y is near 1 keeps
       // its small loss instead of the fp32 rounding of lse itself (the one-pass path's M = e_n also cancels)
-      const float d = (M - xy[n]) + ls;
+      const float d = (M - xt) + ls;
       if (gate == nullptr) {
         // plain cross-entropy: loss = lse - x_y; a target outside [0, V_real) (xy = -inf) is ignored.
         // (loss_rows == nullptr: only lse is wanted.)
-        const bool ok = xy[n] != -INFINITY;
+        const bool ok = xt != -INFINITY;
         loss = ok ? d : 0.f;
         wgt = ok ? 1.f : 0.f;
         if (loss_rows != nullptr) {
@@ -1328,7 +1463,14 @@ __global__ __launch_bounds__(256) void k_fwd_merge(const float* __restrict__ par
         wgt_rows[n] = wgt;
         dgr_rows[n] = clamped ? 0.f : (py - h) / Pc;
       }
-      if (tr.G != nullptr) train_row(tr, n, wgt, M + ls, xy[n]);
+      if (tr.G != nullptr) train_row(tr, n, wgt, M + ls, xt);
+    }
+    if constexpr (RB == 64) {  // one wave holds the block's rows (a single block)
+      if (loss_sum != nullptr) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
+        if (t == 0) loss_sum[0] = loss;
+      }
     }
   }
 }
@@ -2991,32 +3133,54 @@ int launch_exact(const uint16_t* H, int64_t ldh, const uint16_t* W, int64_t ldw,
   return launch_status();
 }
 
-// The forward kernels: row logits (xy, and the candidate logits), tiles, merge (and, with a sparse bias, the exact
-// pass). Outputs the merge does not need to write may be null (loss_rows with wgt_rows, dgr_rows).
+// The forward kernels: with a sparse bias the row logits (xy and the candidate logits; otherwise the tiles give xy and
+// the merge -inf for the targets they have not), tiles, merge (and, with a sparse bias, the exact pass). Outputs the
+// merge does not need to write may be null (loss_rows with wgt_rows, dgr_rows). loss_sum not null: the sum of loss_rows.
+int launch_merge(const FwdWs& w, const int64_t* y, float* xy, int kc, const float* gate, const float* hit, int64_t N,
+                 int64_t grid_rows, int T, int64_t V_real, float* loss_rows, float* lse_rows, float* wgt_rows,
+                 float* dgr_rows, int* xcount, const TrainRows& tr, float* loss_sum, hipStream_t st) {
+  if (grid_rows <= NARROW_ROWS)
+    hipLaunchKernelGGL((k_fwd_merge<64, 1024>), dim3(1), dim3(1024), 0, st, w.part_m, w.part_s, xy, w.cb, w.xc, kc, gate,
+                       hit, N, T, loss_rows, lse_rows, wgt_rows, dgr_rows, xcount, w.xlist, tr, y, V_real, loss_sum);
+  else
+    hipLaunchKernelGGL((k_fwd_merge<32, 256>), dim3((unsigned)cdiv(grid_rows, 32)), dim3(256), 0, st, w.part_m, w.part_s,
+                       xy, w.cb, w.xc, kc, gate, hit, N, T, loss_rows, lse_rows, wgt_rows, dgr_rows, xcount, w.xlist,
+                       tr, y, V_real, nullptr);
+  return launch_status();
+}
+
 int fwd_launch(const FwdWs& w, const uint16_t* H, int64_t ldh, const uint16_t* W, int64_t ldw, const float* bias,
                const int64_t* y, const float* gate, const float* hit, const int64_t* cand, const float* cval, int kc,
                int64_t N, int64_t K, int64_t V, int64_t V_real, float* xy, float* loss_rows, float* lse_rows,
-               float* wgt_rows, float* dgr_rows, hipStream_t st) {
+               float* wgt_rows, float* dgr_rows, float* loss_sum, hipStream_t st) {
   int rc;
   const int tv = (int)cdiv(V, BM), tn = (int)cdiv(N, BN);
   const Operand Wop{W, ldw, V, K, 0}, Hop{H, ldh, N, K, 0};
-  hipLaunchKernelGGL(k_row_logits, dim3((unsigned)cdiv(N, 4)), dim3(256), 0, st, H, ldh, W, ldw, bias, y, cand, cval,
-                     kc, N, K, V_real, xy, w.xc, w.cb, w.xcount);
-  if ((rc = launch_status())) return rc;
+  if (kc > 0) {
+    hipLaunchKernelGGL(k_row_logits, dim3((unsigned)cdiv(N, 4)), dim3(256), 0, st, H, ldh, W, ldw, bias, y, cand, cval,
+                       kc, N, K, V_real, xy, w.xc, w.cb, w.xcount);
+    if ((rc = launch_status())) return rc;
+  }
+  // a single-block merge also adds up the losses (with a sparse bias some of them change after it)
+  const bool sums = loss_sum != nullptr && kc == 0 && N <= NARROW_ROWS;
   {
     ProfScope prof(PROF_FWD_TILES, st);
     const TargetArgs ta{y, cand, cval, kc, xy};
-    MCE_LAUNCH_KM(k_fwd_tiles, K, dim3(tv * tn), dim3(NTHREADS), 0, st, Wop, Hop, bias, N, V, V_real, tv, tn,
-                  w.part_m, w.part_s, ta);
+    if (N <= NARROW_ROWS)
+      hipLaunchKernelGGL(k_fwd_narrow, dim3(2 * tv), dim3(NTHREADS), 0, st, Wop, Hop, bias, N, V, V_real, w.part_m,
+                         w.part_s, ta);
+    else
+      MCE_LAUNCH_KM(k_fwd_tiles, K, dim3(tv * tn), dim3(NTHREADS), 0, st, Wop, Hop, bias, N, V, V_real, tv, tn,
+                    w.part_m, w.part_s, ta);
   }
   if ((rc = launch_status())) return rc;
-  hipLaunchKernelGGL(k_fwd_merge, dim3((unsigned)cdiv(N, 32)), dim3(256), 0, st, w.part_m, w.part_s, xy, w.cb, w.xc,
-                     kc, gate, hit, N, 2 * tv, loss_rows, lse_rows, wgt_rows, dgr_rows, kc > 0 ? w.xcount : nullptr, w.xlist,
-                     TrainRows{});
-  if ((rc = launch_status())) return rc;
-  if (kc == 0) return MCE_OK;
-  return launch_exact(H, ldh, W, ldw, bias, cand, cval, kc, N, K, V, V_real, tv, w.xcount, w.xlist, w.part_m,
-                      w.part_s, xy, loss_rows, lse_rows, wgt_rows, st);
+  if ((rc = launch_merge(w, kc > 0 ? nullptr : y, xy, kc, gate, hit, N, N, 2 * tv, V_real, loss_rows, lse_rows, wgt_rows,
+                         dgr_rows, kc > 0 ? w.xcount : nullptr, TrainRows{}, sums ? loss_sum : nullptr, st)))
+    return rc;
+  if (kc > 0 && (rc = launch_exact(H, ldh, W, ldw, bias, cand, cval, kc, N, K, V, V_real, tv, w.xcount, w.xlist,
+                                   w.part_m, w.part_s, xy, loss_rows, lse_rows, wgt_rows, st)))
+    return rc;
+  return loss_sum != nullptr && !sums ? launch_sum(loss_rows, N, w.sum_part, loss_sum, st) : MCE_OK;
 }
 
 // Forward of every variant: gate and hit both given (mixture) or both null (plain cross-entropy); kc sparse
@@ -3038,10 +3202,8 @@ int fwd_impl(const uint16_t* H, int64_t ldh, const uint16_t* W, int64_t ldw, con
   if (!y || !loss_rows || !lse_rows || !wgt_rows || (gate && !dgr_rows) || !ws) return MCE_EINVAL;
   const FwdWs w = fwd_ws_layout(reinterpret_cast<char*>(ws), N, V, kc);
   if (ws_bytes < w.bytes) return MCE_EWORKSPACE;
-  if ((rc = fwd_launch(w, H, ldh, W, ldw, bias, y, gate, hit, cand, cval, kc, N, K, V, V_real, w.xy, loss_rows,
-                       lse_rows, wgt_rows, dgr_rows, st)))
-    return rc;
-  return launch_sum(loss_rows, N, w.sum_part, loss_sum, st);
+  return fwd_launch(w, H, ldh, W, ldw, bias, y, gate, hit, cand, cval, kc, N, K, V, V_real, w.xy, loss_rows, lse_rows,
+                    wgt_rows, dgr_rows, loss_sum, st);
 }
 
 // The logits-gradient kernels of every variant on a laid-out backward workspace: G of the N rows into w.G, plus
@@ -3448,11 +3610,16 @@ int fwd_train_impl(const uint16_t* H, int64_t ldh, uint16_t* W, int64_t ldw, con
     int* xcount = w.counts + w.np / BLK + b;
     const TrainRows tr{y + row0, w.lse_est + row0, w.flag + row0, rp, V_real, w.arow + row0, w.counts + b, w.flag_list,
                        w.G};
-    hipLaunchKernelGGL(k_fwd_merge, dim3((unsigned)(rp / 32)), dim3(256), 0, st, w.part_m, w.part_s, w.xy + row0,
-                       w.cb + row0 * kc, w.xc + row0 * kc, kc, at(gate, row0), at(hit, row0), rows, 2 * tv,
-                       loss_rows + row0, lse_rows + row0, wgt_rows + row0, at(dgr_rows, row0),
-                       kc > 0 ? xcount : nullptr, w.xlist, kc > 0 ? TrainRows{} : tr);
-    if ((rc = launch_status())) return rc;
+    FwdWs mw{};
+    mw.part_m = w.part_m;
+    mw.part_s = w.part_s;
+    mw.xc = w.xc + row0 * kc;
+    mw.cb = w.cb + row0 * kc;
+    mw.xlist = w.xlist;
+    if ((rc = launch_merge(mw, nullptr, w.xy + row0, kc, at(gate, row0), at(hit, row0), rows, rp, 2 * tv, V_real,
+                           loss_rows + row0, lse_rows + row0, wgt_rows + row0, at(dgr_rows, row0),
+                           kc > 0 ? xcount : nullptr, kc > 0 ? TrainRows{} : tr, nullptr, st)))
+      return rc;
     if (kc > 0) {
       if ((rc = launch_exact(H + row0 * ldh, ldh, W, ldw, bias, at(cand, row0 * kc), at(cval, row0 * kc), kc, rows, K,
                              V, V_real, tv, xcount, w.xlist, w.part_m, w.part_s, w.xy + row0, loss_rows + row0,
@@ -3691,7 +3858,7 @@ int mce_lse_fwd(const uint16_t* H, int64_t ldh, const uint16_t* W, int64_t ldw, 
   const FwdWs w = fwd_ws_layout(reinterpret_cast<char*>(ws), N, V, 0);
   if (ws_bytes < w.bytes) return MCE_EWORKSPACE;
   return fwd_launch(w, H, ldh, W, ldw, bias, y, nullptr, nullptr, nullptr, nullptr, 0, N, K, V, V_real, ly_rows,
-                    nullptr, lse_rows, nullptr, nullptr, reinterpret_cast<hipStream_t>(stream));
+                    nullptr, lse_rows, nullptr, nullptr, nullptr, reinterpret_cast<hipStream_t>(stream));
 }
 
 int mce_bwd_lse_grad(const uint16_t* H, int64_t ldh, const uint16_t* W, int64_t ldw, const float* bias,

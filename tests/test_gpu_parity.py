@@ -243,3 +243,50 @@ def test_mixed_input_dtypes(path, monkeypatch):
     got = dict(loss=float(loss.detach()), dh=h.grad.float().cpu().numpy(), dw=w.grad.float().cpu().numpy(),
                dgate=g.grad.float().cpu().numpy())
     assert_parity(got, fwd, bwd, f"mixed dtypes {path}")
+
+
+@pytest.mark.parametrize("N", [1, 31, 32, 33, 63, 64, 65, 129])
+@pytest.mark.parametrize("K,V,vr", [(64, 100, None), (72, 128, 127), (200, 129, None), (1040, 3001, 2900), (2048, 385, 257)])
+@pytest.mark.parametrize("mode", ["mix", "ce", "sparse"])
+def test_statistics_of_few_rows(mode, N, K, V, vr):
+    """The statistics pass at its row limits (64 rows: the narrow tiles and the single-block merge; 65 and more: the
+    whole tiles), ragged K and V, a vocabulary ending inside a 128-row tile, masked ids, and, without the row-logits
+    pass (all but the sparse bias), targets outside the vocabulary. lse and loss are fp32 sums of K products: 1e-5."""
+    from memarch_amd import fused_ops
+    print(f"few rows {mode} N={N} K={K} V={V} vr={vr}", flush=True)
+    c = random_case(N, K, V, vr, True, seed=N + K + V)
+    y = c["y"].clone()
+    if mode != "mix":
+        y[::5] = -100
+        if vr is not None:
+            y[3::7] = vr
+    gate, hit = (c["gate"], c["hit"]) if mode == "mix" else (None, None)
+    sp = {}
+    if mode == "sparse":
+        g = torch.Generator().manual_seed(N)
+        sp = dict(cand=torch.randint(0, V, (N, 3), generator=g), cval=torch.randn(N, 3, generator=g))
+    dev = lambda t: None if t is None else t.cuda()  # noqa: E731
+    r = fused_ops.forward_rows(c["h"].cuda().bfloat16(), c["w"].cuda(), y.cuda(), dev(gate), dev(hit),
+                               bias=c["bias"].cuda(), v_real=vr, **{k: v.cuda() for k, v in sp.items()})
+    n = lambda t: None if t is None else t.numpy()  # noqa: E731
+    ref = orc.forward(orc.bf16_round(c["h"].numpy()), orc.bf16_round(c["w"].numpy()), y.numpy(), n(gate), n(hit),
+                      c["bias"].numpy(), vr, cand=n(sp.get("cand")), cval=n(sp.get("cval")))
+    np.testing.assert_allclose(r["lse"].cpu().numpy(), ref["lse"], rtol=1e-5, atol=1e-5)
+    np.testing.assert_allclose(r["loss_rows"].cpu().numpy(), ref["loss_rows"], rtol=1e-4, atol=1e-5)
+    np.testing.assert_allclose(r["wgt"].cpu().numpy(), ref["wgt"], rtol=1e-4, atol=1e-5)
+    assert abs(float(r["loss_sum"]) - ref["loss_rows"].sum()) <= 1e-5 * max(1.0, np.abs(ref["loss_rows"]).sum())
+
+
+@pytest.mark.parametrize("N", [5, 64, 300])
+def test_lse_forward_targets_outside(N, monkeypatch):
+    """chunk_ce's statistics forward writes ly = -inf itself for targets the tiles do not hold."""
+    from memarch_amd import chunk_ce, fused_ops
+    monkeypatch.setattr(fused_ops, "RECOMPUTE", True)
+    c = random_case(N, 128, 700, None, True, seed=N)
+    y = c["y"].clone()
+    y[::3] = -1
+    lse, ly = chunk_ce.chunk_ce(c["h"].cuda().bfloat16().requires_grad_(), c["w"].cuda(), c["bias"].cuda(), y.cuda())
+    ref = orc.forward(orc.bf16_round(c["h"].numpy()), orc.bf16_round(c["w"].numpy()), y.numpy(), None, None,
+                      c["bias"].numpy())
+    np.testing.assert_allclose(lse.detach().cpu().numpy(), ref["lse"], rtol=1e-5, atol=1e-5)
+    np.testing.assert_allclose(ly.detach().cpu().numpy(), ref["xy"], rtol=1e-4, atol=1e-4)
