@@ -60,7 +60,8 @@ class _ChunkCE(torch.autograd.Function):
         ctx.train = None
         if _one_pass(n, kp, v, want):
             (hd, wd, bf, y64, _, _), rows, _, _, state = fused_ops._fwd_launch(h, W, b, y, None, None, v,
-                                                                              train=True, want=want)
+                                                                              train=True, want=want,
+                                                                              own_rows=True)
             lse = rows["lse"]
             ly = torch.empty(n, dtype=torch.float32, device=dev)
             _lib.call("mce_train_target_logits", _ptr(state["ws"]), n, kp, v, state["block_rows"], _ptr(ly),

@@ -37,7 +37,8 @@ FLAGGED = None
 
 
 def _stream(dev):
-    return torch.cuda.current_stream(dev).cuda_stream
+    """torch's current stream of the device, as the pointer the library takes (without building a Stream object)."""
+    return torch._C._cuda_getCurrentRawStream(dev.index)
 
 
 def _ptr(t):
@@ -77,7 +78,15 @@ def _bf16_operand(t, kp):
 
 
 def _rows(t, dtype):
+    if t.dtype is dtype and t.dim() == 1 and t.is_contiguous():
+        return t
     return t.detach().reshape(-1).to(dtype).contiguous()
+
+
+def _row_ptrs(rows):
+    """Addresses of the loss, lse, wgt and dgr rows of a training forward's per-row buffer."""
+    p, s = rows.data_ptr(), 4 * rows.shape[1]
+    return p, p + s, p + 2 * s, p + 3 * s
 
 
 def _check_sparse(cand, cval, n, gate):
@@ -96,11 +105,13 @@ def _check_sparse(cand, cval, n, gate):
     return kc
 
 
-def _fwd_launch(h, w, bias, y, gate, hit, v_real, cand=None, cval=None, train=False, want=0):
+def _fwd_launch(h, w, bias, y, gate, hit, v_real, cand=None, cval=None, train=False, want=0,
+                own_rows=False):
     """Validates the inputs, prepares the bf16 operands and runs mce_fwd (or mce_fwd_sparse when a sparse bias
     cand/cval [N, k] is given, or for train=True the one-pass mce_fwd_train / mce_fwd_train_sparse, forming the
-    gradients `want` names, GRAD_* bits) on the current stream. Returns (operands, per-row outputs, loss_sum, meta, training state or
-    None); the training state holds the workspace and the partial sums of the gradients the backward completes."""
+    gradients `want` names, GRAD_* bits) on the current stream. Returns (operands, per-row outputs, loss_sum, meta,
+    training state or None). The per-row outputs are a dict of tensors, or for train=True (without own_rows) one buffer (_row_ptrs); the
+    training state holds the workspace and the partial sums of the gradients the backward completes."""
     if h.dim() != 2 or w.dim() != 2 or h.shape[1] != w.shape[1]:
         raise ValueError(f"h {tuple(h.shape)} and w {tuple(w.shape)} must be [N, K] and [V, K]")
     n, k = h.shape
@@ -134,9 +145,16 @@ def _fwd_launch(h, w, bias, y, gate, hit, v_real, cand=None, cval=None, train=Fa
     if kc:
         cand64, cval32 = cand.detach().to(torch.int64).contiguous(), cval.detach().to(torch.float32).contiguous()
     f32 = dict(dtype=torch.float32, device=dev)
-    loss_rows, lse, wgt, dgr = (torch.empty(n, **f32) for _ in range(4))
     loss_sum = torch.empty((), **f32)
     lib = _lib.load()
+    if train and not own_rows:
+        # the per-row outputs go no further than the backward: one buffer, read through its rows' addresses
+        rows = torch.empty(4, (n + 63) // 64 * 64, **f32)
+        p_loss, p_lse, p_wgt, p_dgr = _row_ptrs(rows)
+    else:
+        loss_rows, lse, wgt, dgr = (torch.empty(n, **f32) for _ in range(4))
+        rows = dict(loss_rows=loss_rows, lse=lse, wgt=wgt, dgr=dgr)
+        p_loss, p_lse, p_wgt, p_dgr = loss_rows.data_ptr(), lse.data_ptr(), wgt.data_ptr(), dgr.data_ptr()
     if train:
         if bf is None:
             want &= ~GRAD_BIAS
@@ -157,34 +175,31 @@ def _fwd_launch(h, w, bias, y, gate, hit, v_real, cand=None, cval=None, train=Fa
         if kc:
             _lib.call("mce_fwd_train_sparse", _ptr(hd), hd.stride(0), _ptr(wd), wd.stride(0), _ptr(w32),
                       0 if w32 is None else w32.stride(0), _ptr(bf), _ptr(y64),
-                      _ptr(cand64), _ptr(cval32), kc, n, kp, v, v_real, BLOCK_ROWS, want, _ptr(loss_rows), _ptr(lse),
-                      _ptr(wgt), _ptr(loss_sum), pd, int(dh_bf16), kp, pw, kp, pb, _ptr(tws), ws_bytes,
+                      _ptr(cand64), _ptr(cval32), kc, n, kp, v, v_real, BLOCK_ROWS, want, p_loss, p_lse,
+                      p_wgt, _ptr(loss_sum), pd, int(dh_bf16), kp, pw, kp, pb, _ptr(tws), ws_bytes,
                       _stream(dev))
-            dgr.zero_()
         else:
             _lib.call("mce_fwd_train", _ptr(hd), hd.stride(0), _ptr(wd), wd.stride(0), _ptr(w32),
                       0 if w32 is None else w32.stride(0), _ptr(bf), _ptr(y64), _ptr(gf),
-                      _ptr(hf), n, kp, v, v_real, BLOCK_ROWS, want, _ptr(loss_rows), _ptr(lse), _ptr(wgt), _ptr(dgr),
+                      _ptr(hf), n, kp, v, v_real, BLOCK_ROWS, want, p_loss, p_lse, p_wgt, p_dgr,
                       _ptr(loss_sum), pd, int(dh_bf16), kp, pw, kp, pb, _ptr(tws), ws_bytes, _stream(dev))
         if FLAGGED is not None and n > 0:
             cnt = torch.empty(1, dtype=torch.int32, device=dev)
             _lib.call("mce_train_flagged", _ptr(tws), n, kp, v, BLOCK_ROWS, _ptr(cnt), _stream(dev))
             FLAGGED.add_(cnt)
-        rows = dict(loss_rows=loss_rows, lse=lse, wgt=wgt, dgr=dgr)
         state = dict(ws=tws, want=want, block_rows=BLOCK_ROWS, dh_bf16=dh_bf16, **parts)
         return (hd, wd, bf, y64, cand64, cval32), rows, loss_sum, (n, k, kp, v, v_real), state
     ws_bytes = lib.mce_fwd_ws_bytes(n, kp, v)
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
     if cand64 is not None:
         _lib.call("mce_fwd_sparse", _ptr(hd), hd.stride(0), _ptr(wd), wd.stride(0), _ptr(bf), _ptr(y64),
-                  _ptr(cand64), _ptr(cval32), kc, n, kp, v, v_real, _ptr(loss_rows), _ptr(lse), _ptr(wgt),
+                  _ptr(cand64), _ptr(cval32), kc, n, kp, v, v_real, p_loss, p_lse, p_wgt,
                   _ptr(loss_sum), _ptr(ws), ws_bytes, _stream(dev))
         dgr.zero_()
     else:
         _lib.call("mce_fwd", _ptr(hd), hd.stride(0), _ptr(wd), wd.stride(0), _ptr(bf), _ptr(y64), _ptr(gf),
-                  _ptr(hf), n, kp, v, v_real, _ptr(loss_rows), _ptr(lse), _ptr(wgt), _ptr(dgr), _ptr(loss_sum),
+                  _ptr(hf), n, kp, v, v_real, p_loss, p_lse, p_wgt, p_dgr, _ptr(loss_sum),
                   _ptr(ws), ws_bytes, _stream(dev))
-    rows = dict(loss_rows=loss_rows, lse=lse, wgt=wgt, dgr=dgr)
     return (hd, wd, bf, y64, cand64, cval32), rows, loss_sum, (n, k, kp, v, v_real), None
 
 
@@ -198,9 +213,11 @@ def _forward(ctx, h, w, bias, y, gate, hit, v_real, cand=None, cval=None):
                                                                           else 0)
     (hd, wd, bf, y64, c64, cv32), rows, loss_sum, meta, state = _fwd_launch(h, w, bias, y, gate, hit, v_real, cand,
                                                                             cval, train, want)
-    # the one-pass backward needs no W (its W^T copy is in the workspace)
-    ctx.save_for_backward(hd, None if state is not None else wd, bf, y64, rows["lse"], rows["wgt"], rows["dgr"], c64,
-                          cv32)
+    if state is not None:
+        # the one-pass backward needs no W (its W^T copy is in the workspace)
+        ctx.save_for_backward(hd, None, bf, y64, rows, None, None, c64, cv32)
+    else:
+        ctx.save_for_backward(hd, wd, bf, y64, rows["lse"], rows["wgt"], rows["dgr"], c64, cv32)
     ctx.train = state   # the one-pass path's workspace and partial sums, read by the backward (None: recompute)
     ctx.meta = meta
     ctx.dtypes = (h.dtype, w.dtype, None if gate is None else gate.dtype, None if bias is None else bias.dtype,
@@ -208,12 +225,21 @@ def _forward(ctx, h, w, bias, y, gate, hit, v_real, cand=None, cval=None):
     return loss_sum
 
 
+# A tensor that already has the shape goes as it is: a reshape would put a node of its own into the backward.
+def _vec(t):
+    return t if t.dim() == 1 else t.reshape(-1)
+
+
+def _mat(t):
+    return t if t.dim() == 2 else t.reshape(-1, t.shape[-1])
+
+
 def _flat(t):
-    return None if t is None else t.reshape(-1)
+    return None if t is None else _vec(t)
 
 
 def _flat_k(t):
-    return None if t is None else t.reshape(-1, t.shape[-1])
+    return None if t is None else _mat(t)
 
 
 @torch.no_grad()
@@ -221,9 +247,16 @@ def forward_rows(h, w, y, gate, hit, bias=None, v_real=None, cand=None, cval=Non
     """The forward pass without autograd: dict of the fp32 loss sum and the per-row loss, lse (logsumexp of the
     row's logits), wgt = (1-g)py/P and dgr = (py-hit)/P (both 0 for rows under the 1e-30 clamp). gate = hit =
     None is plain cross-entropy (wgt = 1, dgr = 0), optionally with a sparse bias cand/cval [..., k]."""
-    _, rows, loss_sum, _, _ = _fwd_launch(h.reshape(-1, h.shape[-1]), w, bias, y.reshape(-1), _flat(gate),
-                                          _flat(hit), v_real, _flat_k(cand), _flat_k(cval))
+    _, rows, loss_sum, _, _ = _fwd_launch(_mat(h), w, bias, _vec(y), _flat(gate), _flat(hit), v_real, _flat_k(cand),
+                                          _flat_k(cval))
     return dict(loss_sum=loss_sum, **rows)
+
+
+def _grad(t, k, dtype):
+    """The first k columns of a gradient in the input's dtype."""
+    if t.shape[1] != k:
+        t = t[:, :k]
+    return t if t.dtype is dtype else t.to(dtype)
 
 
 def _backward(ctx, go, need_h, need_w, need_b, need_g, need_c=False):
@@ -232,7 +265,7 @@ def _backward(ctx, go, need_h, need_w, need_b, need_g, need_c=False):
     n, k, kp, v, v_real = ctx.meta
     hdt, wdt, gdt, bdt, cdt = ctx.dtypes
     dev = hd.device
-    go32 = go.detach().reshape(()).to(torch.float32).contiguous()
+    go32 = go if go.dtype is torch.float32 and go.dim() == 0 else go.detach().reshape(()).to(torch.float32).contiguous()
     f32 = dict(dtype=torch.float32, device=dev)
     dgate = torch.empty(n, **f32) if need_g else None
     dbias = torch.empty(v, **f32) if (need_b and bf is not None) else None
@@ -241,6 +274,7 @@ def _backward(ctx, go, need_h, need_w, need_b, need_g, need_c=False):
     state = getattr(ctx, "train", None)
     if state is not None:
         st = _stream(dev)
+        _, p_lse, p_wgt, p_dgr = _row_ptrs(lse)
         tws, want = state["ws"], state["want"]
         nb = tws.numel()
         need_h, need_w = need_h and bool(want & GRAD_H), need_w and bool(want & GRAD_W)
@@ -248,16 +282,16 @@ def _backward(ctx, go, need_h, need_w, need_b, need_g, need_c=False):
             dbias = None
         dhf = torch.empty(n, kp, dtype=_BF16 if state["dh_bf16"] else torch.float32, device=dev) if need_h else None
         dwf = torch.empty(v, kp, **f32) if need_w else None
-        _lib.call("mce_bwd_train", _ptr(hd), hd.stride(0), _ptr(go32), _ptr(dgr), n, kp, v, state["block_rows"],
+        _lib.call("mce_bwd_train", _ptr(hd), hd.stride(0), _ptr(go32), p_dgr, n, kp, v, state["block_rows"],
                   _ptr(state["dh"]) if need_h else None, _ptr(state["dw"]) if need_w else None,
                   _ptr(state["dbias"]) if dbias is not None else None, _ptr(dhf), int(state["dh_bf16"]), kp,
                   _ptr(dwf), kp, _ptr(dbias), _ptr(dgate), _ptr(tws), nb, st)
         if need_h:
-            dh = dhf[:, :k].to(hdt)
+            dh = _grad(dhf, k, hdt)
         if need_w:
-            dw = dwf[:, :k].to(wdt)
+            dw = _grad(dwf, k, wdt)
         if dcval is not None:
-            _lib.call("mce_bwd_train_dcval", _ptr(y64), _ptr(c64), _ptr(cv32), c64.shape[1], _ptr(lse), _ptr(wgt),
+            _lib.call("mce_bwd_train_dcval", _ptr(y64), _ptr(c64), _ptr(cv32), c64.shape[1], p_lse, p_wgt,
                       _ptr(go32), n, kp, v, v_real, state["block_rows"], _ptr(dcval), _ptr(tws), nb, st)
     elif need_h or need_w or need_g or dbias is not None or dcval is not None:
         # the recompute backward, block by block (its workspace bounded by one block of rows)
@@ -273,9 +307,9 @@ def _backward(ctx, go, need_h, need_w, need_b, need_g, need_c=False):
                   _ptr(go32), n, kp, v, v_real, BLOCK_ROWS, _ptr(dhf), int(out_bf16), kp, _ptr(dwf), kp,
                   _ptr(dbias), _ptr(dgate), _ptr(dcval), _ptr(ws), ws_bytes, _stream(dev))
         if need_h:
-            dh = dhf[:, :k].to(hdt)
+            dh = _grad(dhf, k, hdt)
         if need_w:
-            dw = dwf[:, :k].to(wdt)
+            dw = _grad(dwf, k, wdt)
     if dgate is not None:
         dgate = dgate.to(gdt)
     if dbias is not None:
@@ -349,20 +383,19 @@ class _LinearCEMixBiased(torch.autograd.Function):
 @torch.compiler.disable
 def linear_ce_mix(h, w, y, gate, hit, chunk=4096):
     """Sum over rows of -log max((1-g)*softmax(h w^T)[y] + g*hit, 1e-30) (fused_ops.py:165-167)."""
-    return _LinearCEMix.apply(h.reshape(-1, h.shape[-1]), w, y.reshape(-1), gate.reshape(-1), hit.reshape(-1), chunk)
+    return _LinearCEMix.apply(_mat(h), w, _vec(y), _vec(gate), _vec(hit), chunk)
 
 
 @torch.compiler.disable
 def linear_ce(h, w, y, chunk=4096):
     """Sum over rows of cross-entropy of logits h w^T against y, logits never stored (fused_ops.py:170-172)."""
-    return _LinearCE.apply(h.reshape(-1, h.shape[-1]), w, y.reshape(-1), chunk)
+    return _LinearCE.apply(_mat(h), w, _vec(y), chunk)
 
 
 @torch.compiler.disable
 def linear_ce_sparse(h, w, y, cand, b, chunk=4096):
     """linear_ce with the sparse logit bias logits[n, cand[n, j]] += b[n, j], j < k <= 64 (fused_ops.py:99-101)."""
-    return _LinearCESparse.apply(h.reshape(-1, h.shape[-1]), w, y.reshape(-1),
-                                 cand.reshape(-1, cand.shape[-1]).long(), b.reshape(-1, b.shape[-1]), chunk)
+    return _LinearCESparse.apply(_mat(h), w, _vec(y), _mat(cand).long(), _mat(b), chunk)
 
 
 @torch.compiler.disable
@@ -370,8 +403,7 @@ def linear_ce_mix_biased(h, w, bias, y, gate, hit, v_real=None, chunk=4096):
     """linear_ce_mix with logits h w^T + bias (fp32) and ids >= v_real masked out; also returns dBias. gate and
     hit may both be None (plain cross-entropy)."""
     del chunk
-    return _LinearCEMixBiased.apply(h.reshape(-1, h.shape[-1]), w, bias, y.reshape(-1), _flat(gate), _flat(hit),
-                                    v_real)
+    return _LinearCEMixBiased.apply(_mat(h), w, bias, _vec(y), _flat(gate), _flat(hit), v_real)
 
 
 def __getattr__(name):

@@ -11,7 +11,7 @@ reference computes it with per-text argsorts on host threads (`prep`, fastloop.p
 import torch
 
 from . import _lib
-from .fused_ops import _check_cuda, _ptr, _stream
+from .fused_ops import _check_cuda, _ptr, _rows, _stream
 
 _LONG_MAX = 1 << 24  # longest text of mce_induct_ws
 
@@ -27,8 +27,8 @@ def _launch(x, locks, longest, bucket, c1_none, want):
         raise ValueError(f"texts of at most {_LONG_MAX} tokens are supported, got T={T}")
     _check_cuda(x, bucket)
     dev = x.device
-    xl = x.detach().to(torch.int64).contiguous()
-    bl = None if bucket is None else bucket.detach().reshape(-1).to(torch.int64).contiguous()
+    xl = x if x.dtype is torch.int64 and x.is_contiguous() else x.detach().to(torch.int64).contiguous()
+    bl = None if bucket is None else _rows(bucket, torch.int64)
     i64 = dict(dtype=torch.int64, device=dev)
     out = dict(cand=torch.empty(B, T, locks, **i64) if "cand" in want else None,
                on=torch.empty(B, T, locks, dtype=torch.bool, device=dev) if "on" in want else None,

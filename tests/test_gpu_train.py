@@ -394,3 +394,28 @@ def test_extra_columns_inside_the_tiles(shape, path, monkeypatch):
         x = K % 256
         for key in ("dh", "dw"):
             assert orc.rel_fro(got[key][:, K - x:], bwd[key][:, K - x:]) <= GRAD_RTOL, (key, "extra columns")
+
+
+@pytest.mark.parametrize("kind", ["mix", "sparse"])
+def test_saved_tensors_on_the_host(kind):
+    """The per-row buffer of a training forward goes through save_for_backward like the operands, so saved-tensor hooks
+    that move it away and back leave the gradients as they are."""
+    from memarch_amd import fused_ops
+    c = random_case(200, 136, 600, None, False, seed=3)
+    h, w, gate = c["h"].cuda().bfloat16().requires_grad_(), c["w"].cuda().requires_grad_(), c["gate"].cuda().requires_grad_()
+    y, hit = c["y"].cuda(), c["hit"].cuda()
+    cand = torch.stack([y, (y + 1) % 600], 1)
+    b = torch.linspace(-1, 1, 400, device="cuda").reshape(200, 2).requires_grad_()
+
+    def grads():
+        if kind == "mix":
+            loss, wrt = fused_ops.linear_ce_mix(h, w, y, gate, hit), (h, w, gate)
+        else:
+            loss, wrt = fused_ops.linear_ce_sparse(h, w, y, cand, b), (h, w, b)
+        return torch.autograd.grad(loss, wrt)
+
+    want = grads()
+    with torch.autograd.graph.save_on_cpu():
+        got = grads()
+    for a, r in zip(got, want):
+        assert torch.equal(a, r)

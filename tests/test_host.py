@@ -123,3 +123,29 @@ def test_reference_module_surface():
     from memarch_amd.fused_ops import swiglu, _SwiGLU  # noqa: F401
     from memarch_amd import swiglu as sw
     assert mod.swiglu is sw.swiglu and mod._SwiGLU is sw._SwiGLU
+
+
+@pytest.mark.parametrize("make", [lambda: torch.arange(12), lambda: torch.arange(12).reshape(3, 4),
+                                  lambda: torch.arange(24)[::2], lambda: torch.arange(12, dtype=torch.int32),
+                                  lambda: torch.arange(12).reshape(3, 4).t(), lambda: torch.tensor(5),
+                                  lambda: torch.zeros(0, dtype=torch.int64), lambda: torch.arange(3).expand(4, 3)])
+def test_row_operands_without_a_copy(make):
+    """_rows passes a contiguous 1-D tensor of the dtype as it is and gives the general path's values for any other;
+    _vec and _mat reshape only what has another shape."""
+    from memarch_amd import fused_ops
+    t = make()
+    r = fused_ops._rows(t, torch.int64)
+    assert torch.equal(r, t.detach().reshape(-1).to(torch.int64).contiguous()) and r.is_contiguous()
+    assert (r is t) == (t.dim() == 1 and t.dtype == torch.int64 and t.is_contiguous())
+    assert torch.equal(fused_ops._vec(t), t.reshape(-1)) and (fused_ops._vec(t) is t) == (t.dim() == 1)
+    if t.dim() > 0 and t.numel():
+        assert torch.equal(fused_ops._mat(t), t.reshape(-1, t.shape[-1])) and (fused_ops._mat(t) is t) == (t.dim() == 2)
+
+
+def test_mixture_still_needs_gate_and_hit():
+    """linear_ce_mix takes no None (linear_ce_mix_biased does)."""
+    from memarch_amd import fused_ops
+    h, w, y, g = torch.zeros(2, 8), torch.zeros(4, 8), torch.zeros(2, dtype=torch.int64), torch.zeros(2)
+    for args in ((h, w, y, None, g), (h, w, y, g, None), (h, w, None, g, g), (None, w, y, g, g)):
+        with pytest.raises(AttributeError):
+            fused_ops.linear_ce_mix(*args)
