@@ -419,3 +419,39 @@ def test_saved_tensors_on_the_host(kind):
         got = grads()
     for a, r in zip(got, want):
         assert torch.equal(a, r)
+
+
+@pytest.mark.parametrize("N,K,V", [(70, 264, 515), (2048, 264, 515), (2049, 264, 515), (2112, 1040, 300), (130, 2056, 257)])
+@pytest.mark.parametrize("lddw_pad,offset", [(0, 0), (4, 0), (8, 4), (1, 0), (0, 1), (2, 0)])
+def test_dw_stores_of_any_stride_and_alignment(N, K, V, lddw_pad, offset):
+    """dW goes out in whole 16-byte units where its rows allow it, and value by value for any other row stride or base
+    (through the C ABI); both leave the columns between K and the row stride alone, with short reductions (non-temporal
+    stores) and longer ones, and with partial sums of an earlier block added."""
+    from memarch_amd import _lib
+    print(f"dW stores N={N} K={K} V={V} pad={lddw_pad} offset={offset}", flush=True)
+    lib = _lib.load()
+    c = random_case(N, K, V, None, False, seed=N + K)
+    go = 1.0 / N
+    fwd, bwd = oracle_of(c, go=go)
+    h, w = c["h"].cuda().bfloat16(), c["w"].cuda().bfloat16()
+    y, gate, hit = c["y"].cuda(), c["gate"].cuda(), c["hit"].cuda()
+    f32 = dict(dtype=torch.float32, device="cuda")
+    p = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    st = torch.cuda.current_stream().cuda_stream
+    ld = K + lddw_pad
+    for block_rows in (0, 1024 if N > 1024 else 256):
+        nb = lib.mce_train_ws_bytes(N, K, V, block_rows)
+        r = (-(-N // lib.mce_train_block_rows(N, K, V, block_rows)) - 1) * lib.mce_train_block_rows(N, K, V, block_rows)
+        ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+        rows = [torch.empty(N, **f32) for _ in range(4)]
+        loss = torch.empty((), **f32)
+        buf = torch.full((V * ld + 8,), 7.5, **f32)
+        dw = buf[offset:offset + V * ld]
+        _lib.call("mce_fwd_train", p(h), K, p(w), K, None, 0, None, p(y), p(gate), p(hit), N, K, V, V, block_rows, 2,
+                  *(p(t) for t in rows), p(loss), None, 1, K, p(dw) if r else None, ld, None, p(ws), nb, st)
+        gt = torch.full((), go, **f32)
+        _lib.call("mce_bwd_train", p(h), K, p(gt), p(rows[3]), N, K, V, block_rows, None, p(dw) if r else None, None, None,
+                  1, K, p(dw), ld, None, None, p(ws), nb, st)
+        got = dw.view(V, ld).cpu().numpy()
+        assert orc.rel_fro(got[:, :K], bwd["dw"]) <= GRAD_RTOL
+        assert (got[:, K:] == 7.5).all() and (buf[:offset] == 7.5).all() and (buf[offset + V * ld:] == 7.5).all()
