@@ -438,7 +438,7 @@ def bench_induct(args):
         "data": f"synthetic (seeded config {cfg.index} token texts)",
         "config": {"workload": f"_induct_raw on config {cfg.index}'s texts", "texts": int(x.shape[0]),
                    "seq": int(x.shape[1]), "locks": 3},
-        "roofline": {"bound": "hbm", "kernel": "k_induct" if x.shape[1] <= 8192 else "k_ind_link",
+        "roofline": {"bound": "hbm", "kernel": "k_induct" if x.shape[1] <= 8192 else "k_ind_insert",
                      "achieved": round(nbytes / dt / 1e9, 2),
                      "peak": PEAK_HBM / 1e9, "unit": "GB/s", "frac": round(nbytes / dt / PEAK_HBM, 6),
                      "bytes_per_launch": nbytes, "traffic": None,

@@ -17,15 +17,15 @@
 //      reads it (the previous position, in an earlier chunk), its last lane writes it. A wave's LDS accesses execute
 //      in order, so the walk does not wait for a chunk's reads before the next chunk's: every lane reads and writes,
 //      the ones with nothing to do at a spare entry of their own, since a branch around an access would wait for it.
-// The work is linear in T; the time is the walk (0.06 us per chunk, 0.11 in the long path) and the latencies of the steps around it.
+// The work is linear in T; the time is the walk (0.06 us per chunk, 0.03 with the infos of PACK texts, 0.11 in longer ones) and the latencies of the steps around it.
 //   k_induct       T <= 8192: one workgroup per text, tables in LDS (16-bit entries), all locks at once up to 2048
 //                  tokens, one after the other above.
 //   k_ind_*        longer texts, T up to 2^24, on a caller-sized workspace: the insert of all locks and texts over the
-//                  whole GPU on tables in global memory, then the walks (LDS holds the latest positions, 147 KB of
-//                  slots per workgroup; a text with more slots takes several workgroups that each keep to their own
-//                  slots), then the outputs.
+//                  whole GPU on tables in global memory, then the walks with the latest positions in LDS (k_ind_walk
+//                  up to 32768 positions; k_ind_link above: a text with more slots than a workgroup's LDS holds takes
+//                  several workgroups that each keep to their own slots), then the outputs.
 // Measured (3 locks): 32 texts x 1024 tokens 12.3 us, 59.6 with the bitonic sorts this replaced; 4 x 8192 81 us against
-// 440; 4 x 16384 62 us (insert 21, walks 34) against 1082; 1 x 2^20 1.65 ms against 143.
+// 440; 4 x 16384 40 us (insert 22, walks 9; k_ind_link walks them in 34) against 1082; 1 x 2^20 1.65 ms against 143.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -217,6 +217,13 @@ constexpr int LINK_THREADS = 256, LONG_AHEAD = 32;
 // Info of a position: its slot plus one (at most 2^25 - 1), bit 25 set for the last lane of its key in the chunk, the
 // lane of the previous position with its key in the chunk (its own lane: none) in bits 26-31; 0 for t < k.
 constexpr uint32_t SLOT_MASK = (1u << 25) - 1;
+// Texts of at most PACK_T positions, whose slots fit in 16 bits, have the two table indexes of the walk instead (the
+// walk is bound by its instructions, and these need none to be worked out): in the low half the entry to read, the slot
+// for the first lane of its key in the chunk, else slots + the lane of the previous position with its key in the chunk
+// (its own lane: none), a spare entry; in the high half the entry to write, the slot for the last lane, else the lane's
+// spare entry. The links then hold what the walk read, and k_ind_emit takes the rest from the infos.
+constexpr int64_t PACK_T = 32768;
+constexpr size_t PACK_SLOTS = 65536 - 64;
 
 // Workspace of one text: the locks' tables, `slots` 32-bit entries each, from the start of the text's part (later
 // the links last[locks][T] i32: the tables are then no longer needed), and the infos [locks][T] u32 at `info`.
@@ -239,7 +246,7 @@ LongLayout long_layout(int64_t T, int locks) {
   l.info = tables;
   l.bytes = tables + align256(4 * (size_t)locks * (size_t)T);
   const size_t slots = std::min(2 * tp, tables / (4 * (size_t)locks));
-  l.slots = (uint32_t)std::min(slots, (size_t)SLOT_MASK - 1);
+  l.slots = (uint32_t)std::min(slots, T <= PACK_T ? PACK_SLOTS : (size_t)SLOT_MASK - 1);
   return l;
 }
 
@@ -273,9 +280,10 @@ __device__ __forceinline__ uint32_t global_slot(uint32_t* tab, uint32_t slots, u
   }
 }
 
-// The infos: a wave per (chunk, lock), 4 chunks per block; block (chunk group * locks + lock, text). Lanes that start
+// The infos (PACK: of texts of at most PACK_T positions): a wave per (chunk, lock), 4 chunks per block; block (chunk group * locks + lock, text). Lanes that start
 // at the same slot let the lowest of them go first and take its slot where their key is the same, so that a frequent
 // key costs one access of its entry per chunk.
+template <bool PACK>
 __global__ __launch_bounds__(256) void k_ind_insert(const int64_t* __restrict__ x, int T, int locks, int bits,
                                                     char* __restrict__ ws, size_t per_text, size_t off_info,
                                                     uint32_t slots) {
@@ -299,7 +307,12 @@ __global__ __launch_bounds__(256) void k_ind_insert(const int64_t* __restrict__ 
   if (__builtin_amdgcn_ballot_w64(ok && !same) != 0) m = match_lanes(s, bits, valid);
   const uint64_t below = m & ((uint64_t(1) << lane) - 1);
   const int prev = below != 0 ? high_bit(below) : lane;
-  if (t < T) info[t] = ok ? (s + 1) | ((m >> lane) == 1 ? 1u << 25 : 0u) | ((uint32_t)prev << 26) : 0u;
+  if (t >= T) return;
+  const bool final = ok && (m >> lane) == 1;
+  if constexpr (PACK)
+    info[t] = (ok && below == 0 ? s : slots + (ok ? prev : lane)) | ((final ? s : slots + lane) << 16);
+  else
+    info[t] = ok ? (s + 1) | (final ? 1u << 25 : 0u) | ((uint32_t)prev << 26) : 0u;
 }
 
 // A 32-bit word at byte offset `off` of a buffer of `bytes` bytes: out-of-range offsets load 0 and store nothing, so a
@@ -309,7 +322,47 @@ __device__ __forceinline__ Rsrc make_rsrc(void* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(p, 0, (int)bytes, 0x00020000);
 }
 
-// The walks: block (part * locks + lock, text) links the positions whose slots are in [part * CAP, (part + 1) * CAP).
+// The walk of a PACK text: block (lock, text); its first wave goes through the chunks, LONG_AHEAD at a time, the infos
+// of the next ones in flight.
+__global__ __launch_bounds__(LINK_THREADS) void k_ind_walk(int T, char* __restrict__ ws, size_t per_text,
+                                                           size_t off_info, uint32_t slots) {
+  __shared__ __attribute__((aligned(16))) uint16_t latest[PACK_SLOTS + 64];
+  const size_t k = blockIdx.x;
+  char* base = ws + (size_t)blockIdx.y * per_text;
+  const Rsrc info = make_rsrc(base + off_info + 4 * k * T, 4 * (uint32_t)T);
+  const Rsrc link = make_rsrc(base + 4 * k * T, 4 * (uint32_t)T);
+  for (uint32_t i = threadIdx.x; i < (slots + 7) / 8; i += LINK_THREADS)
+    reinterpret_cast<uint4*>(latest)[i] = uint4{NONE32, NONE32, NONE32, NONE32};
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  const int lane = threadIdx.x, nch = (T + 63) >> 6;
+  const uint32_t idle = (slots + lane) * 0x10001u;  // past the text: nothing to read or write
+  uint32_t nx[LONG_AHEAD];
+#pragma unroll
+  for (int u = 0; u < LONG_AHEAD; ++u) nx[u] = __builtin_amdgcn_raw_buffer_load_b32(info, lane * 4, u * 256, 0);
+  for (int c0 = 0; c0 < nch; c0 += LONG_AHEAD) {
+    uint32_t f[LONG_AHEAD], l[LONG_AHEAD];
+#pragma unroll
+    for (int u = 0; u < LONG_AHEAD; ++u) {
+      f[u] = nx[u];
+      nx[u] = __builtin_amdgcn_raw_buffer_load_b32(info, lane * 4, (c0 + LONG_AHEAD + u) * 256, 0);
+    }
+    if ((c0 + LONG_AHEAD) * 64 > T) {  // the last batch
+#pragma unroll
+      for (int u = 0; u < LONG_AHEAD; ++u)
+        if ((c0 + u) * 64 + lane >= T) f[u] = idle;
+    }
+#pragma unroll
+    for (int u = 0; u < LONG_AHEAD; ++u) {
+      l[u] = latest[f[u] & 0xFFFFu];
+      latest[f[u] >> 16] = (uint16_t)((c0 + u) * 64 + lane);
+    }
+#pragma unroll
+    for (int u = 0; u < LONG_AHEAD; ++u) __builtin_amdgcn_raw_buffer_store_b32(l[u], link, lane * 4, (c0 + u) * 256, 0);
+  }
+}
+
+// The walks of longer texts: block (part * locks + lock, text) links the positions whose slots are in [part * CAP, (part + 1) * CAP).
 // P: the type of a position (16 bits while every position and the empty mark fit). The first wave walks; the infos of
 // the next LONG_AHEAD chunks are loaded before a batch of chunks is walked, so that the walk (about 0.06 us per chunk)
 // covers their latency.
@@ -358,16 +411,28 @@ __global__ __launch_bounds__(LINK_THREADS) void k_ind_link(int T, int locks, cha
   }
 }
 
+template <bool PACK>
 __global__ __launch_bounds__(256) void k_ind_emit(const int64_t* __restrict__ x, int T, int locks, int longest,
                                                   const int64_t* __restrict__ bucket, int64_t nbucket, int64_t c1_none,
                                                   const char* __restrict__ ws, size_t per_text,
                                                   int64_t* __restrict__ cand, uint8_t* __restrict__ on,
                                                   int64_t* __restrict__ src, int64_t* __restrict__ bk,
-                                                  int64_t* __restrict__ c1, int64_t text0) {
+                                                  int64_t* __restrict__ c1, int64_t text0, size_t off_info,
+                                                  uint32_t slots) {
   const int32_t* last = reinterpret_cast<const int32_t*>(ws + (size_t)blockIdx.y * per_text);
+  const uint32_t* info = reinterpret_cast<const uint32_t*>(ws + (size_t)blockIdx.y * per_text + off_info);
   const int64_t row0 = (text0 + blockIdx.y) * T;
   emit(x + (int64_t)blockIdx.y * T, row0, T, locks, longest,
-       [&](int k, int t) { return (int)last[(size_t)k * T + t]; }, bucket, nbucket, c1_none, cand, on, src, bk, c1,
+       [&](int k, int t) {
+         const int l = last[(size_t)k * T + t];
+         if constexpr (PACK) {
+           const uint32_t f = info[(size_t)k * T + t] & 0xFFFFu;
+           if (f < slots) return l == (int)NONE16 ? -1 : l;
+           return (int)(f - slots) == (t & 63) ? -1 : (t & ~63) + (int)(f - slots);
+         }
+         return l;
+       },
+       bucket, nbucket, c1_none, cand, on, src, bk, c1,
        (int)blockIdx.x * 256 + (int)threadIdx.x, (int)gridDim.x * 256);
 }
 
@@ -442,18 +507,31 @@ int mce_induct_ws(const int64_t* x, int64_t B, int64_t T, int locks, int longest
     hipLaunchKernelGGL(k_ind_clear, dim3(std::min(1024u, (entries + 1023) / 1024), nb), dim3(256), 0, st, w, l.bytes,
                        entries);
     if ((rc = launched())) return rc;
-    hipLaunchKernelGGL(k_ind_insert, dim3(groups * (unsigned)locks, nb), dim3(256), 0, st, x + b0 * T, (int)T, locks,
-                       bits, w, l.bytes, l.info, l.slots);
+    const dim3 igrid(groups * (unsigned)locks, nb), egrid(std::min(4096u, groups), nb);
+    const int64_t* xb = x + b0 * T;
+    const int tt = (int)T, lo = longest ? 1 : 0;
+    if (T <= PACK_T) {
+      hipLaunchKernelGGL((k_ind_insert<true>), igrid, dim3(256), 0, st, xb, tt, locks, bits, w, l.bytes, l.info, l.slots);
+      if ((rc = launched())) return rc;
+      hipLaunchKernelGGL(k_ind_walk, dim3((unsigned)locks, nb), dim3(LINK_THREADS), 0, st, tt, w, l.bytes, l.info,
+                         l.slots);
+      if ((rc = launched())) return rc;
+      hipLaunchKernelGGL((k_ind_emit<true>), egrid, dim3(256), 0, st, xb, tt, locks, lo, bucket, nbucket, c1_none, w,
+                         l.bytes, cand, on, src, bk, c1, b0, l.info, l.slots);
+      if ((rc = launched())) return rc;
+      continue;
+    }
+    hipLaunchKernelGGL((k_ind_insert<false>), igrid, dim3(256), 0, st, xb, tt, locks, bits, w, l.bytes, l.info, l.slots);
     if ((rc = launched())) return rc;
     if (small)
-      hipLaunchKernelGGL((k_ind_link<uint16_t>), dim3(parts * (unsigned)locks, nb), dim3(LINK_THREADS), 0, st,
-                         (int)T, locks, w, l.bytes, l.info);
+      hipLaunchKernelGGL((k_ind_link<uint16_t>), dim3(parts * (unsigned)locks, nb), dim3(LINK_THREADS), 0, st, tt, locks,
+                         w, l.bytes, l.info);
     else
-      hipLaunchKernelGGL((k_ind_link<uint32_t>), dim3(parts * (unsigned)locks, nb), dim3(LINK_THREADS), 0, st,
-                         (int)T, locks, w, l.bytes, l.info);
+      hipLaunchKernelGGL((k_ind_link<uint32_t>), dim3(parts * (unsigned)locks, nb), dim3(LINK_THREADS), 0, st, tt, locks,
+                         w, l.bytes, l.info);
     if ((rc = launched())) return rc;
-    hipLaunchKernelGGL(k_ind_emit, dim3(std::min(4096u, groups), nb), dim3(256), 0, st, x + b0 * T, (int)T, locks,
-                       longest ? 1 : 0, bucket, nbucket, c1_none, w, l.bytes, cand, on, src, bk, c1, b0);
+    hipLaunchKernelGGL((k_ind_emit<false>), egrid, dim3(256), 0, st, xb, tt, locks, lo, bucket, nbucket, c1_none, w,
+                       l.bytes, cand, on, src, bk, c1, b0, l.info, l.slots);
     if ((rc = launched())) return rc;
   }
   return MCE_INDUCT_OK;

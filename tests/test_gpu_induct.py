@@ -175,11 +175,12 @@ def _edge_texts(kind, B, T, seed):
     return pool[np.tile(r.integers(0, 64, (B, 61)), (1, T // 61 + 1))[:, :T]]
 
 
-@pytest.mark.parametrize("T", [3, 63, 65, 129, 2047, 2048, 2049, 4097, 8191, 8193, 16640, 65534, 65535, 73800])
+@pytest.mark.parametrize("T", [3, 63, 65, 129, 2047, 2048, 2049, 4097, 8191, 8193, 16640, 32767, 32768, 32769, 65534, 65535,
+                               73800])
 @pytest.mark.parametrize("kind", ["one", "two", "distinct", "marked", "wide"])
 def test_table_edges_exact(kind, T):
-    """Chunk remainders (64 positions), the lengths where the kernel, the table or the position type changes (2048,
-    8192, 65535), walks over one and several slot ranges, and texts that fill the hash table least and most."""
+    """Chunk remainders (64 positions), the lengths where the kernel, the table, the info or the position type changes
+    (2048, 8192, 32768, 65535), walks over one and several slot ranges, and texts that fill the hash table least and most."""
     print(f"induct edges {kind} T={T}", flush=True)
     x = _edge_texts(kind, 2, T, T)
     ids, rank = np.unique(x, return_inverse=True)     # the oracle runs on ranks: a relabelling keeps every equality
