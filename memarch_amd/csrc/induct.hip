@@ -25,7 +25,7 @@
 //                  up to 32768 positions; k_ind_link above: a text with more slots than a workgroup's LDS holds takes
 //                  several workgroups that each keep to their own slots), then the outputs.
 // Measured (3 locks): 32 texts x 1024 tokens 12.3 us, 59.6 with the bitonic sorts this replaced; 4 x 8192 81 us against
-// 440; 4 x 16384 40 us (insert 22, walks 9; k_ind_link walks them in 34) against 1082; 1 x 2^20 1.65 ms against 143.
+// 440; 4 x 16384 39 us (insert 22, walks 8; k_ind_link walks them in 34) against 1082; 1 x 2^20 1.65 ms against 143.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -316,7 +316,8 @@ __global__ __launch_bounds__(256) void k_ind_insert(const int64_t* __restrict__ 
 }
 
 // A 32-bit word at byte offset `off` of a buffer of `bytes` bytes: out-of-range offsets load 0 and store nothing, so a
-// walk needs no branch around its accesses.
+// walk needs no branch around its accesses. (The whole offset goes into the per-lane operand: the scalar one is not part
+// of the bounds check.)
 typedef __amdgpu_buffer_rsrc_t Rsrc;
 __device__ __forceinline__ Rsrc make_rsrc(void* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(p, 0, (int)bytes, 0x00020000);
@@ -339,13 +340,13 @@ __global__ __launch_bounds__(LINK_THREADS) void k_ind_walk(int T, char* __restri
   const uint32_t idle = (slots + lane) * 0x10001u;  // past the text: nothing to read or write
   uint32_t nx[LONG_AHEAD];
 #pragma unroll
-  for (int u = 0; u < LONG_AHEAD; ++u) nx[u] = __builtin_amdgcn_raw_buffer_load_b32(info, lane * 4, u * 256, 0);
+  for (int u = 0; u < LONG_AHEAD; ++u) nx[u] = __builtin_amdgcn_raw_buffer_load_b32(info, lane * 4 + u * 256, 0, 0);
   for (int c0 = 0; c0 < nch; c0 += LONG_AHEAD) {
     uint32_t f[LONG_AHEAD], l[LONG_AHEAD];
 #pragma unroll
     for (int u = 0; u < LONG_AHEAD; ++u) {
       f[u] = nx[u];
-      nx[u] = __builtin_amdgcn_raw_buffer_load_b32(info, lane * 4, (c0 + LONG_AHEAD + u) * 256, 0);
+      nx[u] = __builtin_amdgcn_raw_buffer_load_b32(info, lane * 4 + (c0 + LONG_AHEAD + u) * 256, 0, 0);
     }
     if ((c0 + LONG_AHEAD) * 64 > T) {  // the last batch
 #pragma unroll
@@ -358,7 +359,8 @@ __global__ __launch_bounds__(LINK_THREADS) void k_ind_walk(int T, char* __restri
       latest[f[u] >> 16] = (uint16_t)((c0 + u) * 64 + lane);
     }
 #pragma unroll
-    for (int u = 0; u < LONG_AHEAD; ++u) __builtin_amdgcn_raw_buffer_store_b32(l[u], link, lane * 4, (c0 + u) * 256, 0);
+    for (int u = 0; u < LONG_AHEAD; ++u)
+      __builtin_amdgcn_raw_buffer_store_b32(l[u], link, lane * 4 + (c0 + u) * 256, 0, 0);
   }
 }
 
