@@ -1091,7 +1091,8 @@ void k_fwd_narrow(Operand Wop, Operand Hop, const float* __restrict__ bias, int6
     acc[0][r] += b;
     acc[1][r] += b;
   }
-  // the lane holding a row's target writes its logit (plus the row's sparse bias on it, as target_pass)
+  // the lane holding a row's target writes its logit plus the row's sparse bias on it, summed by itself in slot order
+  // as target_pass sums it (added onto the logit one by one, values that cancel would take its low bits along)
 #pragma unroll
   for (int nj = 0; nj < 2; ++nj) {
     const int64_t d = yv[nj] - (v0 + wave * 32) - 4 * lh;
@@ -1100,9 +1101,10 @@ void k_fwd_narrow(Operand Wop, Operand Hop, const float* __restrict__ bias, int6
 #pragma unroll
       for (int r = 0; r < 16; ++r) x = acc_row(0, r, 0) == (int)d ? acc[nj][r] : x;
       const int64_t n = nj * 32 + lr;
+      float by = 0.f;
       for (int k = 0; k < ta.kc; ++k)
-        if (ta.cand[n * ta.kc + k] == yv[nj]) x += ta.cval[n * ta.kc + k];
-      ta.xy[n] = x;
+        if (ta.cand[n * ta.kc + k] == yv[nj]) by += ta.cval[n * ta.kc + k];
+      ta.xy[n] = x + by;
     }
     float m = -INFINITY;
 #pragma unroll

@@ -277,6 +277,26 @@ def test_statistics_of_few_rows(mode, N, K, V, vr):
     assert abs(float(r["loss_sum"]) - ref["loss_rows"].sum()) <= 1e-5 * max(1.0, np.abs(ref["loss_rows"]).sum())
 
 
+@pytest.mark.parametrize("N", [1, 33, 64, 65])
+@pytest.mark.parametrize("big", [1e4, 1e6])
+def test_few_rows_cancelling_biases_on_the_target(N, big):
+    """A target that is repeated among its row's candidates with values that cancel: the values are added up by
+    themselves, in slot order, and only their sum goes onto the logit, so the target's logit keeps its low bits (added
+    one by one they would round it to an ulp of `big`: 0.001 and 0.06). Bounds as in test_statistics_of_few_rows."""
+    from memarch_amd import fused_ops
+    print(f"cancelling biases N={N} big={big}", flush=True)
+    K, V = 200, 385
+    c = random_case(N, K, V, None, True, seed=N)
+    cand = torch.stack([c["y"], c["y"], (c["y"] + 1) % V, c["y"]], 1)
+    cval = torch.tensor([big, -big, 0.5, 0.25]).expand(N, 4).contiguous()
+    r = fused_ops.forward_rows(c["h"].cuda().bfloat16(), c["w"].cuda(), c["y"].cuda(), None, None, bias=c["bias"].cuda(),
+                               cand=cand.cuda(), cval=cval.cuda())
+    ref = orc.forward(orc.bf16_round(c["h"].numpy()), orc.bf16_round(c["w"].numpy()), c["y"].numpy(), None, None,
+                      c["bias"].numpy(), None, cand=cand.numpy(), cval=cval.numpy())
+    np.testing.assert_allclose(r["lse"].cpu().numpy(), ref["lse"], rtol=1e-5, atol=1e-5)
+    np.testing.assert_allclose(r["loss_rows"].cpu().numpy(), ref["loss_rows"], rtol=1e-4, atol=1e-5)
+
+
 @pytest.mark.parametrize("N", [5, 64, 300])
 def test_lse_forward_targets_outside(N, monkeypatch):
     """chunk_ce's statistics forward writes ly = -inf itself for targets the tiles do not hold."""
