@@ -2285,8 +2285,9 @@ void k_exact_train(Operand Wop, const uint16_t* __restrict__ Hf, int64_t K, cons
     }
     // the target and candidate entries of the tile's rows over the stored ones, one thread per row: E'[n, y_n] =
     // exp(x_y - lse_n) - 1 and, for each distinct valid candidate c != y_n, E'[n, c] = exp(x_c + B_c - lse_n), from
-    // the row logits of k_row_logits (x_y with its sparse bias, x_c without)
-    __threadfence();
+    // the row logits of k_row_logits (x_y with its sparse bias, x_c without). Both writers of an entry are threads of
+    // this workgroup, so the barrier orders them; a device-scope fence would write back the XCD's L2 from every wave
+    // (a step of 32768 x 2048 with 30% of the rows flagged: 19.95 ms with it, 18.30 without).
     __syncthreads();
     if (n0 + t >= cnt) return;
     const int64_t n = list[n0 + t], yn = fx.y[n];
