@@ -125,9 +125,9 @@ def _long_texts(seed, B, T, V):
                                    (1, 70000, 50257)], ids=lambda v: str(v))
 @pytest.mark.parametrize("locks,longest", [(3, True), (2, False), (1, True)])
 def test_long_texts_exact(B, T, V, locks, longest):
-    """Texts longer than one workgroup's LDS holds (mce_induct_ws): the sort over the workspace with LDS chunk
-    rounds, up to five wide stages per k at T = 70000 (131072 padded positions), against the argsort oracle; every
-    output bit-exact (cand, on, src, bk, c1)."""
+    """Texts longer than one workgroup's LDS holds (mce_induct_ws): hash tables in the workspace, one walk per text and
+    lock up to 32768 tokens and one per range of slots at T = 70000, against the argsort oracle; every output bit-exact
+    (cand, on, src, bk, c1)."""
     print(f"induct long B={B} T={T} V={V} locks={locks} longest={longest}", flush=True)
     x = _long_texts(B * 31 + T + V, B, T, V)
     bucket = np.arange(40) // 6
@@ -159,7 +159,7 @@ def test_long_texts_large_token_ids():
 def _edge_texts(kind, B, T, seed):
     """one: a single id; two: two ids; distinct: every token once; marked: every other token the same id and the ones
     between all different (long runs of one token whose pairs and triples never repeat); wide: ids over the whole int64
-    range in repeated blocks."""
+    range in repeated blocks, both ends of it and ids that differ in a single one of the top 14 bits among them."""
     r = np.random.default_rng(seed)
     if kind == "one":
         return np.full((B, T), 5, np.int64)
@@ -171,8 +171,13 @@ def _edge_texts(kind, B, T, seed):
         x = np.stack([r.permutation(T) + 1 for _ in range(B)])
         x[:, ::2] = 0
         return x
-    pool = r.integers(-(1 << 49), 1 << 49, 64)
-    return pool[np.tile(r.integers(0, 64, (B, 61)), (1, T // 61 + 1))[:, :T]]
+    lim = np.iinfo(np.int64)
+    base = r.integers(lim.min, lim.max, dtype=np.int64, endpoint=True)
+    top = base ^ (np.uint64(1) << np.arange(50, 64, dtype=np.uint64)).view(np.int64)
+    pool = np.concatenate([[lim.min, lim.max, lim.min + 1, lim.max - 1, 0, -1, base], top,
+                           r.integers(lim.min, lim.max, 43, dtype=np.int64, endpoint=True)])
+    block = np.stack([np.concatenate([r.permutation(len(pool)), r.integers(0, len(pool), 3)]) for _ in range(B)])
+    return pool[np.tile(block, (1, T // block.shape[1] + 1))[:, :T]]
 
 
 @pytest.mark.parametrize("T", [3, 63, 65, 129, 2047, 2048, 2049, 4097, 8191, 8193, 16640, 32767, 32768, 32769, 65534, 65535,

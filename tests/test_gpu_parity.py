@@ -282,7 +282,8 @@ def test_statistics_of_few_rows(mode, N, K, V, vr):
 def test_few_rows_cancelling_biases_on_the_target(N, big):
     """A target that is repeated among its row's candidates with values that cancel: the values are added up by
     themselves, in slot order, and only their sum goes onto the logit, so the target's logit keeps its low bits (added
-    one by one they would round it to an ulp of `big`: 0.001 and 0.06). Bounds as in test_statistics_of_few_rows."""
+    one by one they would round it to an ulp of `big`: 0.001 and 0.06). Logits and losses are below 20 and sums of 200
+    products in fp32: 1e-5 of them."""
     from memarch_amd import fused_ops
     print(f"cancelling biases N={N} big={big}", flush=True)
     K, V = 200, 385
@@ -294,7 +295,7 @@ def test_few_rows_cancelling_biases_on_the_target(N, big):
     ref = orc.forward(orc.bf16_round(c["h"].numpy()), orc.bf16_round(c["w"].numpy()), c["y"].numpy(), None, None,
                       c["bias"].numpy(), None, cand=cand.numpy(), cval=cval.numpy())
     np.testing.assert_allclose(r["lse"].cpu().numpy(), ref["lse"], rtol=1e-5, atol=1e-5)
-    np.testing.assert_allclose(r["loss_rows"].cpu().numpy(), ref["loss_rows"], rtol=1e-4, atol=1e-5)
+    np.testing.assert_allclose(r["loss_rows"].cpu().numpy(), ref["loss_rows"], rtol=1e-5, atol=1e-5)
 
 
 @pytest.mark.parametrize("N", [5, 64, 300])
