@@ -79,6 +79,9 @@ __device__ __forceinline__ uint64_t match_lanes(uint32_t v, int bits, uint64_t v
   return ((uint64_t)hi << 32) | lo;
 }
 __device__ __forceinline__ int high_bit(uint64_t m) { return 63 - __builtin_clzll(m); }
+// Orders this wave's LDS accesses before the call ahead of those after it, where a walk's lanes hand positions to each
+// other: the hardware executes a wave's LDS accesses in order, and this keeps the compiler to it (no instruction).
+__device__ __forceinline__ void wave_lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local"); }
 
 // Outputs of positions i0, i0 + step, ... of a text (xt: its tokens; row0: its first position's flat index) from
 // last_at(k, t), the previous position with t's k-gram or -1. cand, on and src go out flat over (t, k), so that the
@@ -195,7 +198,9 @@ __global__ __launch_bounds__(IND_THREADS_MAX) void k_induct(const int64_t* __res
         for (int u = 0; u < LINK_AHEAD; ++u) {
           const uint32_t s = f[u] & 0x3FFFu;
           r[u] = latest[f[u] & (1u << 14) ? s : 2 * TM + lane];
+          wave_lds_order();
           latest[f[u] & (1u << 15) ? s : 2 * TM + lane] = (uint32_t)((c0 + u) * 64 + lane);
+          wave_lds_order();
         }
 #pragma unroll
         for (int u = 0; u < LINK_AHEAD; ++u)
@@ -356,7 +361,9 @@ __global__ __launch_bounds__(LINK_THREADS) void k_ind_walk(int T, char* __restri
 #pragma unroll
     for (int u = 0; u < LONG_AHEAD; ++u) {
       l[u] = latest[f[u] & 0xFFFFu];
+      wave_lds_order();
       latest[f[u] >> 16] = (uint16_t)((c0 + u) * 64 + lane);
+      wave_lds_order();
     }
 #pragma unroll
     for (int u = 0; u < LONG_AHEAD; ++u)
@@ -399,7 +406,9 @@ __global__ __launch_bounds__(LINK_THREADS) void k_ind_link(int T, int locks, cha
       const uint32_t s = (f[u] & SLOT_MASK) - 1 - lo;
       const bool mine = f[u] != 0 && s < CAP;
       l[u] = latest[mine && (int)(f[u] >> 26) == lane ? s : CAP + lane];
+      wave_lds_order();
       latest[mine && (f[u] & (1u << 25)) ? s : CAP + lane] = (P)((c0 + u) * 64 + lane);
+      wave_lds_order();
     }
 #pragma unroll
     for (int u = 0; u < LA; ++u) {

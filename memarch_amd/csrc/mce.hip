@@ -2469,6 +2469,10 @@ __global__ __launch_bounds__(256) void k_cast_transpose(const float* __restrict_
 // tile (tm, tn < 8) forms them for its row groups as the dot products above are formed, by one MFMA per group and
 // stage, and writes them with the epilogue below; a K-split tail tile writes its slice's values to
 // xpart[((slot * DB + j) * 32 + i) * 32 + n] (row i of group j, extra column n), which xtail_reduce adds up.
+// Orders this wave's LDS accesses before the call ahead of those after it, where lanes of one wave hand values to each
+// other through LDS: the hardware executes a wave's LDS accesses in order, and this keeps the compiler to it (no
+// instruction).
+__device__ __forceinline__ void wave_lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local"); }
 constexpr int NT_STAGES = 32;  // 2048 rows
 template <bool OUT_BF16, bool KF, int AM, int DB, bool XM = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(NTHREADS, NTHREADS), amdgpu_waves_per_eu(1, 1)))
@@ -2594,6 +2598,7 @@ void k_gemm(Operand A, Operand B, int nk_total, int64_t M, int64_t Nc, int tiles
       const int64_t col = n0 + wn * 128 + 4 * lr;
 #pragma unroll
       for (int mh = 0; mh < 2; ++mh) {
+        wave_lds_order();  // the first half's values are read
 #pragma unroll
         for (int q = 0; q < 2; ++q)
 #pragma unroll
@@ -2601,6 +2606,7 @@ void k_gemm(Operand A, Operand B, int nk_total, int64_t M, int64_t Nc, int tiles
 #pragma unroll
             for (int nj = 0; nj < 4; ++nj)
               stage[out_row<AM>(q, r, lh) * 128 + nj * 32 + lr] = acc_read(acc[2 * mh + q][nj][r]);
+        wave_lds_order();  // the half is written
         const int64_t i0 = m0 + wm * 128 + mh * 64 + lh;  // the lane's rows: i0, i0 + 2, ..
         f32x4 cv[32];
         if (cin != nullptr) {  // all of a half's before any of it is stored (Cin may be C itself)
