@@ -2473,7 +2473,6 @@ __global__ __launch_bounds__(256) void k_cast_transpose(const float* __restrict_
 // other through LDS: the hardware executes a wave's LDS accesses in order, and this keeps the compiler to it (no
 // instruction).
 __device__ __forceinline__ void wave_lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local"); }
-constexpr int NT_STAGES = 32;  // 2048 rows
 template <bool OUT_BF16, bool KF, int AM, int DB, bool XM = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(NTHREADS, NTHREADS), amdgpu_waves_per_eu(1, 1)))
 void k_gemm(Operand A, Operand B, int nk_total, int64_t M, int64_t Nc, int tiles_m, int tiles_n, int group,
@@ -2588,8 +2587,7 @@ void k_gemm(Operand A, Operand B, int nk_total, int64_t M, int64_t Nc, int tiles
   // 32 KiB of LDS, so that a lane stores four consecutive columns and an instruction two whole 512-byte row segments. A
   // wave has at most 64 stores in flight, 16 KiB of them when they are single values, and a tile of few K stages then
   // waits for most of its time on stores (dW at K = 2048, V = 50304: 64 rows 126 -> 113 us, 1024 rows 272 -> 254, 32768
-  // unchanged). Up to NT_STAGES stages the stores are also non-temporal, so that they leave the operand panels in the L2
-  // (1024 rows 254 -> 246 us, 256 rows 140 -> 130, 2048 rows 400 -> 395; but 4096 rows 711 -> 740).
+  // unchanged).
   if constexpr (!OUT_BF16) {
     if ((ldc & 3) == 0 && (Nc & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0 &&
         (reinterpret_cast<uintptr_t>(cin) & 15) == 0) {
@@ -2623,12 +2621,7 @@ void k_gemm(Operand A, Operand B, int nk_total, int64_t M, int64_t Nc, int tiles
           if (cin != nullptr) v += cv[i];
           v *= rscale != nullptr ? rs[wm * 128 + mh * 64 + 2 * i + lh] : gs;
           f32x4* dst = reinterpret_cast<f32x4*>(reinterpret_cast<float*>(C) + (i0 + 2 * i) * ldc + col);
-          if (i0 + 2 * i < M && col < Nc) {
-            if (nk_total <= NT_STAGES)
-              __builtin_nontemporal_store(v, dst);
-            else
-              *dst = v;
-          }
+          if (i0 + 2 * i < M && col < Nc) *dst = v;
         }
       }
       return;

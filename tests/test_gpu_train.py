@@ -425,8 +425,8 @@ def test_saved_tensors_on_the_host(kind):
 @pytest.mark.parametrize("lddw_pad,offset", [(0, 0), (4, 0), (8, 4), (1, 0), (0, 1), (2, 0)])
 def test_dw_stores_of_any_stride_and_alignment(N, K, V, lddw_pad, offset):
     """dW goes out in whole 16-byte units where its rows allow it, and value by value for any other row stride or base
-    (through the C ABI); both leave the columns between K and the row stride alone, with short reductions (non-temporal
-    stores) and longer ones, and with partial sums of an earlier block added."""
+    (through the C ABI); both leave the columns between K and the row stride alone, with short reductions and longer
+    ones, and with partial sums of an earlier block added."""
     from memarch_amd import _lib
     print(f"dW stores N={N} K={K} V={V} pad={lddw_pad} offset={offset}", flush=True)
     lib = _lib.load()
