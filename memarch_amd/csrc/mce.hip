@@ -2341,23 +2341,22 @@ __global__ __launch_bounds__(256) void k_dbias_gemv(const uint16_t* __restrict__
 
 // ---------------------------------------------------------------------------------------------------------
 // K-blocked transpose: dst element (c, r) at dst[(r/256)*C*256 + c*256 + kperm(r%256)] = src[r*ld + c] for r < R,
-// 0 for R <= r < (grid rows); c < C (C % 8 == 0). With rscale, source row r is first multiplied by
-// go[0] * rscale[r] (fp32) and rounded to bf16; uperm (needs rscale) then also receives those factors as bf16 in
-// the same kperm order, uperm[p] for every p < grid rows (0 past R). One workgroup per 64 x 64 tile, staged through LDS. The
-// reduction index r is stored in the permuted order kperm that G uses for its vocabulary positions (its 16-byte
-// stores), so the products of the dH contraction (W^T) pair up; natural != 0 stores r (and uperm) in natural order
-// instead, the order of G's rows that the dW contraction reduces over (H^T).
+// 0 for R <= r < (grid rows); c < C (C % 8 == 0). With rscale, source row r is first multiplied by rscale[r] (fp32)
+// and rounded to bf16; urow (needs rscale) then also receives those factors as bf16, urow[r] for every r < grid rows
+// (0 past R). One workgroup per 64 x 64 tile, staged through LDS. The reduction index r is stored in the permuted
+// order kperm that G uses for its vocabulary positions (its 16-byte stores), so the products of the dH contraction
+// (W^T) pair up; natural != 0 stores r in natural order instead, the order of G's rows that the dW contraction reduces
+// over (H^T).
 typedef uint16_t TransposeTile[64][66];
 __device__ __forceinline__ void transpose_tile(const uint16_t* __restrict__ src, int64_t ld, int64_t R, int64_t C,
                                                uint16_t* __restrict__ dst, const float* __restrict__ rscale,
-                                               const float* __restrict__ go, uint16_t* __restrict__ uperm, int natural,
-                                               TransposeTile& tile, int bx, int by) {
+                                               uint16_t* __restrict__ urow, int natural, TransposeTile& tile, int bx,
+                                               int by) {
   const int t = threadIdx.x;
   const int64_t r0 = (int64_t)bx * 64, c0 = (int64_t)by * 64;
-  if (uperm != nullptr && by == 0 && t < 64) {
-    // the row scales themselves, bf16, in the same order: uperm[r0 + p] = go * rscale[r0 + kperm_inv(p)]
-    const int64_t r = r0 + (natural ? t : kperm_inv(t));
-    uperm[r0 + t] = r < R ? to_bf16((go != nullptr ? go[0] : 1.f) * rscale[r]) : (uint16_t)0;
+  if (urow != nullptr && by == 0 && t < 64) {
+    const int64_t r = r0 + t;
+    urow[r] = r < R ? to_bf16(rscale[r]) : (uint16_t)0;
   }
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -2366,8 +2365,8 @@ __device__ __forceinline__ void transpose_tile(const uint16_t* __restrict__ src,
     u16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
     if (r < R && c < C) {
       v = *reinterpret_cast<const u16x8*>(src + r * ld + c);
-      if (rscale != nullptr) {  // row r scaled by go * rscale[r], rounded back to bf16
-        const float f = (go != nullptr ? go[0] : 1.f) * rscale[r];
+      if (rscale != nullptr) {  // row r scaled by rscale[r], rounded back to bf16
+        const float f = rscale[r];
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = to_bf16(f * bf16_to_f32(v[e]));
       }
@@ -2397,12 +2396,9 @@ __device__ __forceinline__ void transpose_tile(const uint16_t* __restrict__ src,
 }
 
 __global__ __launch_bounds__(256) void k_transpose_blocked(const uint16_t* __restrict__ src, int64_t ld, int64_t R,
-                                                           int64_t C, uint16_t* __restrict__ dst,
-                                                           const float* __restrict__ rscale = nullptr,
-                                                           const float* __restrict__ go = nullptr,
-                                                           uint16_t* __restrict__ uperm = nullptr, int natural = 0) {
+                                                           int64_t C, uint16_t* __restrict__ dst, int natural) {
   __shared__ __attribute__((aligned(16))) TransposeTile tile;
-  transpose_tile(src, ld, R, C, dst, rscale, go, uperm, natural, tile, (int)blockIdx.x, (int)blockIdx.y);
+  transpose_tile(src, ld, R, C, dst, nullptr, nullptr, natural, tile, (int)blockIdx.x, (int)blockIdx.y);
 }
 
 // The bf16 cast of an fp32 weight and its K-blocked transpose in one pass: w16[r, c] = bf16(src[r, c]) (round to
@@ -2817,7 +2813,7 @@ struct MidJob {
   int64_t ldh, rows, K;
   uint16_t* Ht;
   const float* rscale;
-  uint16_t* uperm;
+  uint16_t* urow;
   int tr_x, tr_y, gate_blocks;
 };
 template <bool DH_BF16>
@@ -2835,7 +2831,7 @@ __global__ __launch_bounds__(256) void k_grads_mid(MidJob j) {
     return;
   }
   b -= j.gate_blocks;
-  transpose_tile(j.H, j.ldh, j.rows, j.K, j.Ht, j.rscale, nullptr, j.uperm, 1, tile, b % j.tr_x, b / j.tr_x);
+  transpose_tile(j.H, j.ldh, j.rows, j.K, j.Ht, j.rscale, j.urow, 1, tile, b % j.tr_x, b / j.tr_x);
 }
 // After: the dW tail tiles, then dBias.
 __global__ __launch_bounds__(256) void k_grads_end(TailJob dw, BiasJob bias) {
@@ -3375,7 +3371,7 @@ int block_contractions(const BwdWs& w, const uint16_t* H, int64_t ldh, int64_t N
   }
   if (dW == nullptr) return MCE_OK;
   hipLaunchKernelGGL(k_transpose_blocked, dim3((unsigned)(np / 64), (unsigned)cdiv(K, 64)), dim3(256), 0, st, H, ldh,
-                     N, K, w.Ht, nullptr, nullptr, nullptr, 1);
+                     N, K, w.Ht, 1);
   if ((rc = launch_status())) return rc;
   const Operand Aop{w.G, np * BLK, V, np, CM_TILE, 2};
   const Operand Bop{w.Ht, BLK, K, np, K * BLK, 0};
@@ -3412,7 +3408,7 @@ int bwd_blocked_impl(const uint16_t* H, int64_t ldh, const uint16_t* W, int64_t 
   if (dH) {
     // Wt = W^T, K-blocked, once for all blocks
     hipLaunchKernelGGL(k_transpose_blocked, dim3((unsigned)(w.vp / 64), (unsigned)cdiv(K, 64)), dim3(256), 0, st, W,
-                       ldw, V, K, w.Wt);
+                       ldw, V, K, w.Wt, 0);
     if ((rc = launch_status())) return rc;
   }
   for (int64_t row0 = 0; row0 < N; row0 += nb) {
@@ -3439,7 +3435,7 @@ int bwd_blocked_impl(const uint16_t* H, int64_t ldh, const uint16_t* W, int64_t 
 // partials, the dW blocks' dBias partials, the K-split tail tiles and the dBias GEMV partials.
 struct TrainWs {
   int64_t np, vp, nb, nblk;
-  uint16_t *G, *Ht, *uperm, *Wt;
+  uint16_t *G, *Ht, *urow, *Wt;
   float *part_m, *part_s, *xy, *xc, *cb, *lse_est, *arow, *upart, *part, *xpart, *dbias_part, *sum_part;
   int *flag, *flag_list, *counts, *xlist, *olist, *ocount;
   size_t bytes;
@@ -3477,7 +3473,7 @@ TrainWs train_ws_layout(char* base, int64_t N, int64_t K, int64_t V, int64_t req
   };
   w.G = reinterpret_cast<uint16_t*>(take(sizeof(uint16_t) * w.vp * nb));
   w.Ht = reinterpret_cast<uint16_t*>(take(sizeof(uint16_t) * nb * K));
-  w.uperm = reinterpret_cast<uint16_t*>(take(sizeof(uint16_t) * nb));
+  w.urow = reinterpret_cast<uint16_t*>(take(sizeof(uint16_t) * nb));
   w.part_m = reinterpret_cast<float*>(take(sizeof(float) * T * nb));
   w.part_s = reinterpret_cast<float*>(take(sizeof(float) * T * nb));
   w.flag_list = reinterpret_cast<int*>(take(sizeof(int) * nb));
@@ -3548,7 +3544,7 @@ int train_block_grads(const TrainWs& w, int64_t b, const uint16_t* H, int64_t ld
     mid.K = K;
     mid.Ht = w.Ht;
     mid.rscale = w.arow + row0;
-    mid.uperm = dBias ? w.uperm : nullptr;
+    mid.urow = dBias ? w.urow : nullptr;
     mid.tr_x = (int)(rp / 64);
     mid.tr_y = (int)cdiv(K, 64);
   }
@@ -3571,7 +3567,7 @@ int train_block_grads(const TrainWs& w, int64_t b, const uint16_t* H, int64_t ld
     const bool xm = kx > 0 && dBias == nullptr;   // the dBias dot products take the extra-column slot otherwise
     TailJob tail{};
     if ((rc = launch_gemm<false>(Aop, Bop, (int)(rk / BK), V, K, 4, dW, lddw, w.part, st, nullptr, go, dW_in,
-                                 dBias ? w.uperm : nullptr, w.upart, PROF_GEMM_DW, xm ? &Xop : nullptr, w.xpart,
+                                 dBias ? w.urow : nullptr, w.upart, PROF_GEMM_DW, xm ? &Xop : nullptr, w.xpart,
                                  &tail)))
       return rc;
     BiasJob bias{};
@@ -3638,7 +3634,7 @@ int fwd_train_impl(const uint16_t* H, int64_t ldh, uint16_t* W, int64_t ldw, con
     if ((rc = launch_status())) return rc;
   } else if (want & MCE_GRAD_H) {
     hipLaunchKernelGGL(k_transpose_blocked, dim3((unsigned)(w.vp / 64), (unsigned)cdiv(K, 64)), dim3(256), 0, st, W,
-                       ldw, V, K, w.Wt, nullptr, nullptr, nullptr);
+                       ldw, V, K, w.Wt, 0);
     if ((rc = launch_status())) return rc;
   }
   // the target and candidate logits, and e_n (the largest of the row's true logits among them), the cleared flags
@@ -3932,7 +3928,7 @@ int mce_bwd_dhidden(const uint16_t* W, int64_t ldw, int64_t N, int64_t K, int64_
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   // Wt = W^T, K-blocked: element (k, v) at Wt[(v/256)*K*256 + k*256 + v%256], zero for V <= v < Vp
   hipLaunchKernelGGL(k_transpose_blocked, dim3((unsigned)(w.vp / 64), (unsigned)cdiv(K, 64)), dim3(256), 0, st, W,
-                     ldw, V, K, w.Wt);
+                     ldw, V, K, w.Wt, 0);
   if ((rc = launch_status())) return rc;
   // dH[n, k] = sum_v G(n, v) Wt(k, v); G's and Wt's columns V..Vp-1 are zero
   const Operand Aop{w.G, 0, N, w.vp, w.np * BLK, 1};
@@ -3959,7 +3955,7 @@ int mce_bwd_dweight(const uint16_t* H, int64_t ldh, int64_t N, int64_t K, int64_
   if (ws_bytes < w.bytes) return MCE_EWORKSPACE;
   // Ht = H^T, K-blocked: element (k, n) at Ht[(n/256)*K*256 + k*256 + n%256], zero for N <= n < Np
   hipLaunchKernelGGL(k_transpose_blocked, dim3((unsigned)(w.np / 64), (unsigned)cdiv(K, 64)), dim3(256), 0, st, H,
-                     ldh, N, K, w.Ht, nullptr, nullptr, nullptr, 1);
+                     ldh, N, K, w.Ht, 1);
   if ((rc = launch_status())) return rc;
   // dW[v, k] = sum_n G(n, v) Ht(k, n), G read transposed, reduction over the padded n < Np (G's rows and Ht's
   // columns N..Np-1 are zero)
