@@ -8,7 +8,7 @@
 // complete key: it has no last and is no other position's last, so only positions t >= k are entered below.
 //
 // No sort. A hash table gives every key a slot, and "the previous position with the same slot" follows in two steps:
-//   1. insert: each position finds or claims the slot of its key (linear probing; the entry is the claiming position,
+//   1. insert: each position finds or claims the slot of its key (open addressing; the entry is the claiming position,
 //      whose tokens are compared, so a slot stands for exactly one key whatever the hash does; the table has more
 //      slots than positions, so a probe always ends). One wave takes one chunk of 64 consecutive positions: matching
 //      the slots across its lanes (one ballot per slot bit) gives each lane the previous lane with its key and marks
@@ -17,15 +17,19 @@
 //      reads it (the previous position, in an earlier chunk), its last lane writes it. A wave's LDS accesses execute
 //      in order, so the walk does not wait for a chunk's reads before the next chunk's: every lane reads and writes,
 //      the ones with nothing to do at a spare entry of their own, since a branch around an access would wait for it.
-// The work is linear in T; the time is the walk (0.06 us per chunk, 0.03 with the infos of PACK texts, 0.11 in longer ones) and the latencies of the steps around it.
-//   k_induct       T <= 8192: one workgroup per text, tables in LDS (16-bit entries), all locks at once up to 2048
-//                  tokens, one after the other above.
+// The time is the walk (0.06 us per chunk, 0.03 with the infos of PACK texts, 0.11 in longer ones) and the latencies of
+// the steps around it. The work is linear in T up to 32768 tokens, where one walk per lock covers a text; above, every
+// part of k_ind_link walks the whole text and the parts grow with T (about 760 per lock at 2^24), so its work grows
+// with T^2, spread over the GPU: one text of 2^20 1.60 ms, of 2^22 16.6 ms, of 2^24 191 ms (the sorts this replaced
+// took 143, 687 and 3296).
+//   k_induct       T <= 8192: one workgroup per text, tables in LDS (32-bit entries; infos and links of 16 bits), all
+//                  locks at once up to 2048 tokens, one after the other above.
 //   k_ind_*        longer texts, T up to 2^24, on a caller-sized workspace: the insert of all locks and texts over the
 //                  whole GPU on tables in global memory, then the walks with the latest positions in LDS (k_ind_walk
 //                  up to 32768 positions; k_ind_link above: a text with more slots than a workgroup's LDS holds takes
 //                  several workgroups that each keep to their own slots), then the outputs.
-// Measured (3 locks): 32 texts x 1024 tokens 12.3 us, 59.6 with the bitonic sorts this replaced; 4 x 8192 81 us against
-// 440; 4 x 16384 39 us (insert 22, walks 8; k_ind_link walks them in 34) against 1082; 1 x 2^20 1.65 ms against 143.
+// Measured (3 locks): 32 texts x 1024 tokens 12.3 us, 59.6 with the bitonic sorts this replaced; 4 x 8192 84 us against
+// 435; 4 x 16384 39 us (insert 21, walks 8; k_ind_link walks them in 34) against 1082.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -36,7 +40,12 @@
 
 namespace {
 
-constexpr int IND_TMAX = 8192;   // positions per text of k_induct
+// Positions per text of k_induct: what one workgroup's LDS holds. A batch of texts pays for the line there, few long
+// texts do not: 3 locks, us, k_induct against the workspace path at the same lengths (built for the comparison):
+//   texts x 2049    1: 24 / 21   16: 25 / 25   64: 26 / 40     300: 50 / 123
+//   texts x 4096    1: 44 / 23   16: 45 / 33   64: 46 / 68     300: 90 / 238
+//   texts x 8192    1: 83 / 24   16: 85 / 46   64: 87 / 113    128: 90 / 205
+constexpr int IND_TMAX = 8192;
 constexpr int IND_SMALL = 2048;  // up to here all locks' tables fit at once, with the tokens
 constexpr int IND_THREADS_MAX = 1024;
 constexpr int LINK_AHEAD = 8;    // chunks of a walk whose infos and reads are in flight together
@@ -269,8 +278,8 @@ __global__ __launch_bounds__(256) void k_ind_clear(char* __restrict__ ws, size_t
 __device__ __forceinline__ uint32_t place(uint32_t h, uint32_t slots) {
   return (uint32_t)(((uint64_t)h * slots) >> 32);
 }
-__device__ __forceinline__ uint32_t global_slot(uint32_t* tab, uint32_t slots, uint64_t h, const int64_t* __restrict__ x,
-                                                int t, int k) {
+__device__ __forceinline__ uint32_t global_slot(uint32_t* tab, uint32_t slots, uint64_t h,
+                                                const int64_t* __restrict__ x, int t, int k) {
   const uint32_t tag = (uint32_t)(h >> 40) & 0x7Fu, mine = (tag << 24) | (uint32_t)t;
   uint32_t g = (uint32_t)h, s = place(g, slots);
   for (int probe = 0;; ++probe) {
@@ -285,9 +294,9 @@ __device__ __forceinline__ uint32_t global_slot(uint32_t* tab, uint32_t slots, u
   }
 }
 
-// The infos (PACK: of texts of at most PACK_T positions): a wave per (chunk, lock), 4 chunks per block; block (chunk group * locks + lock, text). Lanes that start
-// at the same slot let the lowest of them go first and take its slot where their key is the same, so that a frequent
-// key costs one access of its entry per chunk.
+// The infos (PACK: of texts of at most PACK_T positions): a wave per (chunk, lock), 4 chunks per block; block (chunk
+// group * locks + lock, text). Lanes that start at the same slot let the lowest of them go first and take its slot
+// where their key is the same, so that a frequent key costs one access of its entry per chunk.
 template <bool PACK>
 __global__ __launch_bounds__(256) void k_ind_insert(const int64_t* __restrict__ x, int T, int locks, int bits,
                                                     char* __restrict__ ws, size_t per_text, size_t off_info,
@@ -321,8 +330,8 @@ __global__ __launch_bounds__(256) void k_ind_insert(const int64_t* __restrict__ 
 }
 
 // A 32-bit word at byte offset `off` of a buffer of `bytes` bytes: out-of-range offsets load 0 and store nothing, so a
-// walk needs no branch around its accesses. (The whole offset goes into the per-lane operand: the scalar one is not part
-// of the bounds check.)
+// walk needs no branch around its accesses. (The whole offset goes into the per-lane operand: the scalar one is not
+// part of the bounds check.)
 typedef __amdgpu_buffer_rsrc_t Rsrc;
 __device__ __forceinline__ Rsrc make_rsrc(void* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(p, 0, (int)bytes, 0x00020000);
@@ -371,10 +380,10 @@ __global__ __launch_bounds__(LINK_THREADS) void k_ind_walk(int T, char* __restri
   }
 }
 
-// The walks of longer texts: block (part * locks + lock, text) links the positions whose slots are in [part * CAP, (part + 1) * CAP).
-// P: the type of a position (16 bits while every position and the empty mark fit). The first wave walks; the infos of
-// the next LONG_AHEAD chunks are loaded before a batch of chunks is walked, so that the walk (about 0.06 us per chunk)
-// covers their latency.
+// The walks of longer texts: block (part * locks + lock, text) links the positions whose slots are in
+// [part * CAP, (part + 1) * CAP). P: the type of a position (16 bits while every position and the empty mark fit). The
+// first wave walks; the infos of the next LONG_AHEAD chunks are loaded before a batch of chunks is walked, so that the
+// walk (about 0.06 us per chunk) covers their latency.
 template <typename P>
 __global__ __launch_bounds__(LINK_THREADS) void k_ind_link(int T, int locks, char* __restrict__ ws, size_t per_text,
                                                            size_t off_info) {
@@ -522,7 +531,8 @@ int mce_induct_ws(const int64_t* x, int64_t B, int64_t T, int locks, int longest
     const int64_t* xb = x + b0 * T;
     const int tt = (int)T, lo = longest ? 1 : 0;
     if (T <= PACK_T) {
-      hipLaunchKernelGGL((k_ind_insert<true>), igrid, dim3(256), 0, st, xb, tt, locks, bits, w, l.bytes, l.info, l.slots);
+      hipLaunchKernelGGL((k_ind_insert<true>), igrid, dim3(256), 0, st, xb, tt, locks, bits, w, l.bytes, l.info,
+                         l.slots);
       if ((rc = launched())) return rc;
       hipLaunchKernelGGL(k_ind_walk, dim3((unsigned)locks, nb), dim3(LINK_THREADS), 0, st, tt, w, l.bytes, l.info,
                          l.slots);
@@ -532,14 +542,15 @@ int mce_induct_ws(const int64_t* x, int64_t B, int64_t T, int locks, int longest
       if ((rc = launched())) return rc;
       continue;
     }
-    hipLaunchKernelGGL((k_ind_insert<false>), igrid, dim3(256), 0, st, xb, tt, locks, bits, w, l.bytes, l.info, l.slots);
+    hipLaunchKernelGGL((k_ind_insert<false>), igrid, dim3(256), 0, st, xb, tt, locks, bits, w, l.bytes, l.info,
+                       l.slots);
     if ((rc = launched())) return rc;
     if (small)
-      hipLaunchKernelGGL((k_ind_link<uint16_t>), dim3(parts * (unsigned)locks, nb), dim3(LINK_THREADS), 0, st, tt, locks,
-                         w, l.bytes, l.info);
+      hipLaunchKernelGGL((k_ind_link<uint16_t>), dim3(parts * (unsigned)locks, nb), dim3(LINK_THREADS), 0, st, tt,
+                         locks, w, l.bytes, l.info);
     else
-      hipLaunchKernelGGL((k_ind_link<uint32_t>), dim3(parts * (unsigned)locks, nb), dim3(LINK_THREADS), 0, st, tt, locks,
-                         w, l.bytes, l.info);
+      hipLaunchKernelGGL((k_ind_link<uint32_t>), dim3(parts * (unsigned)locks, nb), dim3(LINK_THREADS), 0, st, tt,
+                         locks, w, l.bytes, l.info);
     if ((rc = launched())) return rc;
     hipLaunchKernelGGL((k_ind_emit<false>), egrid, dim3(256), 0, st, xb, tt, locks, lo, bucket, nbucket, c1_none, w,
                        l.bytes, cand, on, src, bk, c1, b0, l.info, l.slots);

@@ -682,9 +682,10 @@ __device__ __forceinline__ void read_bias_mask(float (&bm)[4][16], const float* 
 // C[m0:m0+256, n0:n0+256] = sum_k A(m, k) B(n, k) over the K stages s0 .. s0+nk-1 (k in [s0*BK, (s0+nk)*BK),
 // clipped to each operand's extent), fp32 accumulation. KF: both operands' K extents are multiples of BK. Either
 // operand may be row-major or K-blocked; A may instead be in the tile-blocked piece layout (Operand::cm = 1), which
-// needs AM = 1 (its LDS image is in piece order), or the transpose of one (Operand::cm = 2, needs AM = 2 and KF). BIAS: A's rows are vocabulary rows and every accumulator starts at its
-// row's bias, masked to -inf for rows >= Vreal (btile: this thread's bias value from tile_bias; bslot: 1 KiB of
-// LDS outside the operand ring), so the epilogue reads the biased, masked logits straight from the accumulators.
+// needs AM = 1 (its LDS image is in piece order), or the transpose of one (Operand::cm = 2, needs AM = 2 and KF).
+// BIAS: A's rows are vocabulary rows and every accumulator starts at its row's bias, masked to -inf for rows >= Vreal
+// (btile: this thread's bias value from tile_bias; bslot: 1 KiB of LDS outside the operand ring), so the epilogue reads
+// the biased, masked logits straight from the accumulators.
 // Output layout (32x32 MFMA): acc[mi][nj][r] is C[wm*128 + mi*32 + 8*(r/4) + 4*(lane/32) + r%4]
 //                                              [wn*128 + nj*32 + lane%32].
 // Two 64 KiB LDS stages, four 16-wide K slices per stage; the fragments of slice kk+1 are read while slice kk is
@@ -1009,6 +1010,10 @@ void k_fwd_tiles(Operand Wop, Operand Hop, const float* __restrict__ bias, int64
 // workgroups leave CUs idle): 64 x 2048 x 50304 takes 48 us against 57 (W alone at the copy rate: 40). K is
 // streamed 64 at a time through three LDS stages of 24 KiB, so that two workgroups of a CU keep up to 144 KiB of loads
 // in flight. Any K; the partials are k_fwd_tiles' (row block = workgroup).
+// The line lies at the 64 columns a tile holds; it is not where the two kernels cross. Whole passes on one W that the
+// caches may hold, us, 1 / 64 rows (this kernel) and 65 / 128 / 256 rows (k_fwd_tiles): 2048 x 50304 41 / 41 and
+// 59 / 56 / 63; 512 x 50304 24 / 23 and 32 / 31 / 32; 2048 x 131072 122 / 121 and 163 / 160 / 171; 256 x 8000 22 / 22
+// and 25 / 25 / 26. A pass with k_fwd_tiles at 1 to 64 rows (and two small launches more): 56-59, 34, 159, 34.
 constexpr int NARROW_ROWS = 64;
 constexpr int NR_V = 128, NR_S = 3, NR_A = NR_V * 128, NR_B = NARROW_ROWS * 128, NR_STAGE = NR_A + NR_B;
 constexpr int NR_LA = NR_A / 4096, NR_LB = NR_B / 4096;  // load instructions per wave and stage
@@ -1021,7 +1026,8 @@ void k_fwd_narrow(Operand Wop, Operand Hop, const float* __restrict__ bias, int6
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int64_t v0 = (int64_t)blockIdx.x * NR_V;
   const int nk = (int)((Wop.kext + BK - 1) / BK);
-  // instruction j < NR_LA: rows 8 (wave*NR_LA + j) .. +7 of W, else of H; lane l: row l/8, 16-byte chunk (l%8) ^ swz(row)
+  // instruction j < NR_LA: rows 8 (wave*NR_LA + j) .. +7 of W, else of H; lane l: row l/8, 16-byte chunk
+  // (l%8) ^ swz(row)
   int voff[NR_LA + NR_LB], kloc[NR_LA + NR_LB];
 #pragma unroll
   for (int j = 0; j < NR_LA + NR_LB; ++j) {
@@ -1340,11 +1346,11 @@ __device__ __forceinline__ bool train_row(const TrainRows& tr, int64_t n, float 
 // negative biases remove nearly all of the sum (a candidate that dominates its row pushed far down), the two would
 // cancel each other and leave rounding noise, so a row whose corrected sum is not above 1/16 of the terms removed is
 // appended to exact_list (its lse, loss and wgt are then rewritten by k_exact_tiles / k_exact_rows).
-// RB rows per block of NT threads, NT / RB threads per row: 32 rows of 256 threads, or, for at most NARROW_ROWS rows, one
-// block of 64 rows and 1024 threads, which leaves each thread a quarter of the folds (a chain of loads and exponentials
-// that is all of such a merge) and can add up the losses itself (loss_sum not null), in a fixed order. (A count of
-// finished blocks would let any number of blocks do so, but its fence writes back the L2 in every block: 60 us instead
-// of 12 for 4096 rows.)
+// RB rows per block of NT threads, NT / RB threads per row: 32 rows of 256 threads, or, for at most NARROW_ROWS rows,
+// one block of 64 rows and 1024 threads, which leaves each thread a quarter of the folds (a chain of loads and
+// exponentials that is all of such a merge) and can add up the losses itself (loss_sum not null), in a fixed order. (A
+// count of finished blocks would let any number of blocks do so, but its fence writes back the L2 in every block: 60 us
+// instead of 12 for 4096 rows.)
 // y not null (the statistics pass without sparse candidates, which forms no row logits): xy holds the targets' logits
 // written by the tiles; a target outside [0, Vreal) gets xy = -inf here.
 template <int RB, int NT>
@@ -2579,11 +2585,11 @@ void k_gemm(Operand A, Operand B, int nk_total, int64_t M, int64_t Nc, int tiles
     rs[t] = i < M ? gs * rscale[i] : 0.f;
     __syncthreads();
   }
-  // fp32 output in whole 16-byte units: each wave turns two halves of its rows (M-subtiles 2mh, 2mh + 1) through its own
-  // 32 KiB of LDS, so that a lane stores four consecutive columns and an instruction two whole 512-byte row segments. A
-  // wave has at most 64 stores in flight, 16 KiB of them when they are single values, and a tile of few K stages then
-  // waits for most of its time on stores (dW at K = 2048, V = 50304: 64 rows 126 -> 113 us, 1024 rows 272 -> 254, 32768
-  // unchanged).
+  // fp32 output in whole 16-byte units: each wave turns two halves of its rows (M-subtiles 2mh, 2mh + 1) through its
+  // own 32 KiB of LDS, so that a lane stores four consecutive columns and an instruction two whole 512-byte row
+  // segments. A wave has at most 64 stores in flight, 16 KiB of them when they are single values, and a tile of few K
+  // stages then waits for most of its time on stores (dW at K = 2048, V = 50304: 64 rows 126 -> 113 us, 1024 rows
+  // 272 -> 254, 32768 unchanged).
   if constexpr (!OUT_BF16) {
     if ((ldc & 3) == 0 && (Nc & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0 &&
         (reinterpret_cast<uintptr_t>(cin) & 15) == 0) {
@@ -2672,8 +2678,8 @@ void k_gemm(Operand A, Operand B, int nk_total, int64_t M, int64_t Nc, int tiles
   }
 }
 
-// The K-split tail tiles of one k_gemm launch (full < tiles_m * tiles_n) and what its epilogue needs; xcols > 0: with the
-// extra columns of its XM mode.
+// The K-split tail tiles of one k_gemm launch (full < tiles_m * tiles_n) and what its epilogue needs; xcols > 0: with
+// the extra columns of its XM mode.
 struct TailJob {
   const float *part, *xpart;
   int P, full, tails, nr, tiles_m, tiles_n, group, am2, xcols;
@@ -3033,8 +3039,8 @@ class ProfScope {
 
 // C = s_i (A . B^T + Cin) over nk stages with the tile grid of k_gemm (s_i, Cin as there). When the tiles leave a
 // partial last wave (or do not fill the GPU once), the R tail tiles are split into P = CUs / R K-slices (at least 2
-// stages each) so the last wave fills the GPU. The tails' reduction is launched here or, with `tail`, left to the caller
-// (no blocks when nothing was split).
+// stages each) so the last wave fills the GPU. The tails' reduction is launched here or, with `tail`, left to the
+// caller (no blocks when nothing was split).
 int launch_status();
 template <bool OUT_BF16>
 int launch_gemm(const Operand& A, const Operand& B, int nk, int64_t M, int64_t Nc, int group, void* C, int64_t ldc,
@@ -3181,22 +3187,25 @@ int launch_exact(const uint16_t* H, int64_t ldh, const uint16_t* W, int64_t ldw,
   return launch_status();
 }
 
-// The forward kernels: with a sparse bias the row logits (xy and the candidate logits; otherwise the tiles give xy and
-// the merge -inf for the targets they have not), tiles, merge (and, with a sparse bias, the exact pass). Outputs the
-// merge does not need to write may be null (loss_rows with wgt_rows, dgr_rows). loss_sum not null: the sum of loss_rows.
+// k_fwd_merge in the shape for grid_rows rows (loss_sum: one block only).
 int launch_merge(const FwdWs& w, const int64_t* y, float* xy, int kc, const float* gate, const float* hit, int64_t N,
                  int64_t grid_rows, int T, int64_t V_real, float* loss_rows, float* lse_rows, float* wgt_rows,
                  float* dgr_rows, int* xcount, const TrainRows& tr, float* loss_sum, hipStream_t st) {
   if (grid_rows <= NARROW_ROWS)
-    hipLaunchKernelGGL((k_fwd_merge<64, 1024>), dim3(1), dim3(1024), 0, st, w.part_m, w.part_s, xy, w.cb, w.xc, kc, gate,
-                       hit, N, T, loss_rows, lse_rows, wgt_rows, dgr_rows, xcount, w.xlist, tr, y, V_real, loss_sum);
+    hipLaunchKernelGGL((k_fwd_merge<64, 1024>), dim3(1), dim3(1024), 0, st, w.part_m, w.part_s, xy, w.cb, w.xc, kc,
+                       gate, hit, N, T, loss_rows, lse_rows, wgt_rows, dgr_rows, xcount, w.xlist, tr, y, V_real,
+                       loss_sum);
   else
-    hipLaunchKernelGGL((k_fwd_merge<32, 256>), dim3((unsigned)cdiv(grid_rows, 32)), dim3(256), 0, st, w.part_m, w.part_s,
-                       xy, w.cb, w.xc, kc, gate, hit, N, T, loss_rows, lse_rows, wgt_rows, dgr_rows, xcount, w.xlist,
-                       tr, y, V_real, nullptr);
+    hipLaunchKernelGGL((k_fwd_merge<32, 256>), dim3((unsigned)cdiv(grid_rows, 32)), dim3(256), 0, st, w.part_m,
+                       w.part_s, xy, w.cb, w.xc, kc, gate, hit, N, T, loss_rows, lse_rows, wgt_rows, dgr_rows, xcount,
+                       w.xlist, tr, y, V_real, nullptr);
   return launch_status();
 }
 
+// The forward kernels: with a sparse bias the row logits (xy and the candidate logits; otherwise the tiles give xy and
+// the merge -inf for the targets they have not), tiles, merge (and, with a sparse bias, the exact pass). Outputs the
+// merge does not need to write may be null (loss_rows with wgt_rows, dgr_rows). loss_sum not null: the sum of
+// loss_rows.
 int fwd_launch(const FwdWs& w, const uint16_t* H, int64_t ldh, const uint16_t* W, int64_t ldw, const float* bias,
                const int64_t* y, const float* gate, const float* hit, const int64_t* cand, const float* cval, int kc,
                int64_t N, int64_t K, int64_t V, int64_t V_real, float* xy, float* loss_rows, float* lse_rows,
@@ -3222,8 +3231,9 @@ int fwd_launch(const FwdWs& w, const uint16_t* H, int64_t ldh, const uint16_t* W
                     w.part_m, w.part_s, ta);
   }
   if ((rc = launch_status())) return rc;
-  if ((rc = launch_merge(w, kc > 0 ? nullptr : y, xy, kc, gate, hit, N, N, 2 * tv, V_real, loss_rows, lse_rows, wgt_rows,
-                         dgr_rows, kc > 0 ? w.xcount : nullptr, TrainRows{}, sums ? loss_sum : nullptr, st)))
+  if ((rc = launch_merge(w, kc > 0 ? nullptr : y, xy, kc, gate, hit, N, N, 2 * tv, V_real, loss_rows, lse_rows,
+                         wgt_rows, dgr_rows, kc > 0 ? w.xcount : nullptr, TrainRows{}, sums ? loss_sum : nullptr,
+                         st)))
     return rc;
   if (kc > 0 && (rc = launch_exact(H, ldh, W, ldw, bias, cand, cval, kc, N, K, V, V_real, tv, w.xcount, w.xlist,
                                    w.part_m, w.part_s, xy, loss_rows, lse_rows, wgt_rows, st)))
@@ -3430,9 +3440,10 @@ int bwd_blocked_impl(const uint16_t* H, int64_t ldh, const uint16_t* W, int64_t 
 
 // Training-path workspace. The rows are processed in blocks of `nb` rows (a multiple of 256; the last block may be
 // shorter): per block E' in G (tile-blocked, the block's rows padded to a multiple of 256), the row-scaled
-// H^T copy and go*a in bf16 (natural row order), the half-tile partials and the flagged-row list, all reused block after
-// block (the last block's stay for the backward); once per call W^T (for dH), the target / candidate logits, e_n, a_n, the flags and the per-block flagged-row counts over all rows, the loss
-// partials, the dW blocks' dBias partials, the K-split tail tiles and the dBias GEMV partials.
+// H^T copy and a in bf16 (natural row order), the half-tile partials and the flagged-row list, all reused block after
+// block (the last block's stay for the backward); once per call W^T (for dH), the target / candidate logits, e_n, a_n,
+// the flags and the per-block flagged-row counts over all rows, the loss partials, the dW blocks' dBias partials, the
+// K-split tail tiles and the dBias GEMV partials.
 struct TrainWs {
   int64_t np, vp, nb, nblk;
   uint16_t *G, *Ht, *urow, *Wt;

@@ -110,8 +110,9 @@ def _fwd_launch(h, w, bias, y, gate, hit, v_real, cand=None, cval=None, train=Fa
     """Validates the inputs, prepares the bf16 operands and runs mce_fwd (or mce_fwd_sparse when a sparse bias
     cand/cval [N, k] is given, or for train=True the one-pass mce_fwd_train / mce_fwd_train_sparse, forming the
     gradients `want` names, GRAD_* bits) on the current stream. Returns (operands, per-row outputs, loss_sum, meta,
-    training state or None). The per-row outputs are a dict of tensors, or for train=True (without own_rows) one buffer (_row_ptrs); the
-    training state holds the workspace and the partial sums of the gradients the backward completes."""
+    training state or None). The per-row outputs are a dict of tensors, or for train=True (without own_rows) one
+    buffer (_row_ptrs); the training state holds the workspace and the partial sums of the gradients the backward
+    completes."""
     if h.dim() != 2 or w.dim() != 2 or h.shape[1] != w.shape[1]:
         raise ValueError(f"h {tuple(h.shape)} and w {tuple(w.shape)} must be [N, K] and [V, K]")
     n, k = h.shape
